@@ -31,7 +31,8 @@ struct DCMarchSampler {
     const int iy = clampi((int)floorf(pos.y), 0, g.gy - 1);
     const int iz = clampi((int)floorf(pos.z), 0, g.gz - 1);
     a.ipos = make_int3(ix, iy, iz);
-    const uint32_t b = findBlock<BW>(g, ix, iy, iz, 0);
+    int lv;
+    const uint32_t b = findBlockLevel<BW>(g, ix, iy, iz, 0, lv);
     if (!precise) {
       const uint32_t c = b * BV + loc<BB>(ix % BW, iy % BW, iz % BW);
 #pragma unroll
@@ -39,16 +40,30 @@ struct DCMarchSampler {
       a.density = (float)g.den[c];
       return;
     }
-    const float scaleInv = 1.f / (float)(1 << g.lev[b]);
+    const float scaleInv = 1.f / (float)(1 << lv);
     const float x = pos.x * scaleInv - .5f, y = pos.y * scaleInv - .5f, z = pos.z * scaleInv - .5f;
     const float xf = floorf(x), yf = floorf(y), zf = floorf(z);
     a.frac = make_float3(x - xf, y - yf, z - zf);
-    const int3 bp = g.pos[b];
+    // the block's level and origin follow from the walk and the cell (no table reads)
+    const int3 bp = make_int3(((ix >> lv) >> BB) << BB, ((iy >> lv) >> BB) << BB, ((iz >> lv) >> BB) << BB);
     const int ai = clampi((int)(xf + 1.f - (float)bp.x), 0, BW);
     const int aj = clampi((int)(yf + 1.f - (float)bp.y), 0, BW);
     const int ak = clampi((int)(zf + 1.f - (float)bp.z), 0, BW);
+    if (ai > 0 && ai < BW && aj > 0 && aj < BW && ak > 0 && ak < BW) {  // all corners in the block
 #pragma unroll
-    for (int k = 0; k < 8; k++) a.cell[k] = apronCell<BW>(g, b, ai + ((k >> 2) & 1), aj + ((k >> 1) & 1), ak + (k & 1));
+      for (int k = 0; k < 8; k++)
+        a.cell[k] = b * BV + loc<BB>(ai - 1 + ((k >> 2) & 1), aj - 1 + ((k >> 1) & 1), ak - 1 + (k & 1));
+    } else {
+      // the corners' descriptors are loaded together (borderApronCell); the block's own entry of
+      // the descriptor table is read but not used
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int ci = ai + ((k >> 2) & 1), cj = aj + ((k >> 1) & 1), ck = ak + (k & 1);
+        const bool own = ci > 0 && ci <= BW && cj > 0 && cj <= BW && ck > 0 && ck <= BW;
+        const uint32_t border = borderApronCell<BW>(g, b, ci, cj, ck);
+        a.cell[k] = own ? b * BV + loc<BB>(ci - 1, cj - 1, ck - 1) : border;
+      }
+    }
     a.density = marchInterp(g.den, a);
   }
   __device__ float3 velocity(const MarchAux& a) const { return marchInterp3(g.vel, a); }
@@ -1080,9 +1095,8 @@ struct DCGridSim : SimBase {
     }
   }
   int render(const dcg_render_params& r, float* rgba) override {
-    const dim3 grid((unsigned)((r.width + 15) / 16), (unsigned)((r.height + 15) / 16));
     DCMarchSampler<BW, DGT<SF>> smp{g};
-    DCG_LAUNCH(DCG_K_OTHER, "k_render", (k_render<<<grid, 256, 0, stream>>>(smp, P, r, (float4*)rgba)));
+    DCG_LAUNCH(DCG_K_OTHER, "k_render", (launchRender(smp, P, r, (float4*)rgba, stream)));
     return DCG_OK;
   }
 

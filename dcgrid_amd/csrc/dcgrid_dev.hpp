@@ -141,9 +141,9 @@ __device__ __forceinline__ int dirIndex(int dx, int dy, int dz) { return (dx + 1
 // per-level hash tables upward from l0; here the walk goes down the child links from the first
 // dense level, which reach exactly the allocated blocks.
 template <int BW>
-__device__ __forceinline__ uint32_t findBlock(const DGBase& g, int qx, int qy, int qz, int l0) {
+__device__ __forceinline__ uint32_t findBlockLevel(const DGBase& g, int qx, int qy, int qz, int l0, int& lv) {
   constexpr int BB = Geo<BW>::BB;
-  int lv = l0 > g.S ? l0 : g.S;
+  lv = l0 > g.S ? l0 : g.S;  // the level of the block found
   int sh = lv - l0;
   const int bx = (qx >> sh) >> BB, by = (qy >> sh) >> BB, bz = (qz >> sh) >> BB;
   uint32_t b = g.offs[lv] + (uint32_t)((bx * g.ry[lv] + by) * g.rz[lv] + bz);
@@ -157,6 +157,11 @@ __device__ __forceinline__ uint32_t findBlock(const DGBase& g, int qx, int qy, i
     lv--;
   }
   return b;
+}
+template <int BW>
+__device__ __forceinline__ uint32_t findBlock(const DGBase& g, int qx, int qy, int qz, int l0) {
+  int lv;
+  return findBlockLevel<BW>(g, qx, qy, qz, l0, lv);
 }
 
 // Neighbour descriptor of one apron direction of a block: x = neighbour block | shift << 27,

@@ -2,7 +2,7 @@
 // (src/fluid_simulation.h:19) for both grids, following src/raymarching.cuh:63-275 with the
 // samplers of src/dcgrid/dcgrid_rendering.cu:6-64 and src/uniformgrid/uniformgrid_rendering.cu:5-47.
 //
-// One thread per pixel in 16x16 tiles. Every float operation is written out in the order of the
+// Sixteen lanes per ray (MarchGroup). Every float operation is written out in the order of the
 // reference's helper_math expressions, with correctly rounded division and square root and the
 // library's own deterministic exp, so the image equals the oracle's restatement bit for bit.
 // Deliberate differences: normalize divides by the length (helper_math multiplies by rsqrtf); the
@@ -13,6 +13,8 @@
 #pragma once
 
 #include <float.h>
+
+#include <utility>
 
 #include "dcg_device.hpp"
 
@@ -106,10 +108,50 @@ __device__ __forceinline__ float3 sceneNormal(const dcg_params& P, float3 p) {
                             sceneSDF(P, make_float3(p.x, p.y, p.z + e)) - sceneSDF(P, make_float3(p.x, p.y, p.z - e))));
 }
 
-// lightmarch (src/raymarching.cuh:80-121)
-template <class S>
-__device__ float lightMarch(const S& smp, const dcg_params& P, const dcg_render_params& R, float3 origin, MarchAux& aux,
-                            float3 sun, float3 sunInv) {
+// The march's lanes per ray. A ray is a long serial chain (up to two samples per cell of its path,
+// each dense one with a shadow march of up to 100 samples), and an image has few rays for this chip:
+// one thread per pixel gives a 256 x 256 image one wavefront per SIMD, bound by the latency of the
+// dependent loads of its slowest ray (the time hardly depended on the resolution). GL = 16 lanes (one
+// DPP row, or a quad of 4) take a ray together: each lane samples its own step of the next GL, and the sums that have to run
+// in the ray's order (positions, optical depth, compositing) are formed by every lane alike from
+// its neighbours' values, in the same order and with the same float operations as by one thread.
+// GL = 1 is the plain loop, for the debug slices (one sample per ray, nothing to share).
+// Measured (MI355X, one thread per ray -> 16 lanes, 256 x 256): plume on the 256^3 grid 34 -> 3.0 ms,
+// on the 512^3 grid 51 -> 3.7 ms, 4^3 blocks with a solid sphere 35 -> 3.2 ms, dense 64^3 grid
+// 1.2 -> 0.30 ms, terrain 2.4 -> 0.72 ms.
+template <int GL>
+struct MarchGroup {
+  static_assert(GL == 1 || GL == 4 || GL == 16, "one thread, one DPP quad or one DPP row per ray");
+  static __device__ __forceinline__ int lane() { return GL == 1 ? 0 : (int)(threadIdx.x & (GL - 1)); }
+  // Value of lane J of the group.
+  template <int J>
+  static __device__ __forceinline__ float from(float v) {
+    if (GL == 1) return v;
+    // quad_perm:[J,J,J,J] or row_newbcast:J; the lanes of a group run the march in lockstep, so
+    // lane J is active
+    constexpr int ctrl = GL == 4 ? 0x55 * J : 0x150 + J;
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xF, 0xF, true));
+  }
+  // Value of lane j, the same j in the whole group.
+  static __device__ __forceinline__ float at(float v, int j) { return GL == 1 ? v : __shfl(v, j, GL); }
+  // Bit k: lane k's condition.
+  static __device__ __forceinline__ uint32_t ballot(bool c) {
+    if (GL == 1) return c ? 1u : 0u;
+    return (uint32_t)(__ballot(c) >> (threadIdx.x & (64u - GL))) & ((1u << GL) - 1u);
+  }
+  // op(J) for J = 0 .. GL - 1, J a constant.
+  template <class Op, int... J>
+  static __device__ __forceinline__ void eachOf(Op op, std::integer_sequence<int, J...>) {
+    (op(std::integral_constant<int, J>{}), ...);
+  }
+  template <class Op>
+  static __device__ __forceinline__ void each(Op op) {
+    eachOf(op, std::make_integer_sequence<int, GL>{});
+  }
+};
+
+// lightmarch (src/raymarching.cuh:80-121), the solid scene's part: 0 = fully shadowed.
+__device__ __forceinline__ float sceneLight(const dcg_params& P, const dcg_render_params& R, float3 origin, float3 sun) {
   float lt = 1.f;
   if (R.solids && P.enable_additional_solids) {
     float dScene = 0.f;
@@ -120,38 +162,115 @@ __device__ float lightMarch(const S& smp, const dcg_params& P, const dcg_render_
       dScene = dScene + sdf;
     }
   }
-  if (R.channel == DCG_RENDER_FLUID) {
-    float dNear, dFar;
-    if (rayDomain(P, dNear, dFar, origin, sunInv)) {
-      float3 pos = origin;
-      if (dNear > 0.f) {
-        pos = v3add(pos, v3mul(sun, dNear));
-        dFar = dFar - dNear;
-      }
-      const float step = fmaxf(dFar / 100.f, 1e-1f);
-      float density = 0.f;
-      for (float d = step; d < dFar && density < 5.f; d = d + step) {
-        pos = v3add(pos, v3mul(sun, step));
-        smp.sample(P, R.precise, pos, aux);
-        density = density + aux.density * P.dx * step;
-      }
-      lt = lt * marchExp(-density);
-    }
-  }
   return lt;
 }
+// lightmarch, the fluid's part, after the scene's `lt`: each lane of the group samples one step.
+template <int GL, class S>
+__device__ __forceinline__ float fluidLight(const S& smp, const dcg_params& P, const dcg_render_params& R, float3 origin,
+                                            float lt, MarchAux& aux, float3 sun, float3 sunInv) {
+  using M = MarchGroup<GL>;
+  if (R.channel != DCG_RENDER_FLUID || lt == 0.f) return lt;
+  float dNear, dFar;
+  if (!rayDomain(P, dNear, dFar, origin, sunInv)) return lt;
+  float3 pos = origin;
+  if (dNear > 0.f) {
+    pos = v3add(pos, v3mul(sun, dNear));
+    dFar = dFar - dNear;
+  }
+  const float step = fmaxf(dFar / 100.f, 1e-1f);
+  const float3 ds = v3mul(sun, step);
+  // the lane's step of the first round: distance and position after lane() + 1 steps
+  const int lane = M::lane();
+  float d = step;
+  pos = v3add(pos, ds);
+  if (GL > 1) {
+#pragma unroll
+    for (int j = 1; j < GL; j++) {
+      const float3 q = v3add(pos, ds);
+      if (lane >= j) {
+        pos = q;
+        d = d + step;
+      }
+    }
+  }
+  float density = 0.f;
+  for (;;) {
+    float c = 0.f;  // adds nothing for a lane past the end
+    if (d < dFar) {
+      smp.sample(P, R.precise, pos, aux);
+      c = aux.density * P.dx * step;
+    }
+    M::each([&](auto J) {
+      const float cj = M::template from<decltype(J)::value>(c);
+      density = density < 5.f ? density + cj : density;
+    });
+    if (!(M::template from<GL - 1>(d) < dFar) || !(density < 5.f)) break;
+#pragma unroll
+    for (int j = 0; j < GL; j++) {
+      pos = v3add(pos, ds);
+      d = d + step;
+    }
+  }
+  return lt * marchExp(-density);
+}
 
-// raymarch (src/raymarching.cuh:123-275); returns (color, alpha).
-template <class S>
-__device__ float4 rayMarch(const S& smp, const dcg_params& P, const dcg_render_params& R, float3 origin, float3 dir,
-                           float3 sun) {
-  enum { NONE, SCENE, FLOOR, DEBUG };
+// What a ray meets behind the fluid (src/raymarching.cuh:144-186), with the solid scene's part of
+// the light there.
+enum : int { MARCH_NONE, MARCH_SCENE, MARCH_FLOOR, MARCH_DEBUG };
+struct MarchSolid {
+  float d;
+  int what;
+  float lt;
+};
+__device__ __forceinline__ MarchSolid marchSolid(const dcg_params& P, const dcg_render_params& R, float3 origin, float3 dir,
+                                                 float3 sun) {
+  const float sliceZ = (float)P.gz * .5f;
+  MarchSolid m{FLT_MAX, MARCH_NONE, 1.f};
+  if (R.channel != DCG_RENDER_FLUID && (sliceZ - origin.z) * dir.z > 0.f) {
+    const float dDebug = (sliceZ - origin.z) / dir.z;
+    const float dx = origin.x + dDebug * dir.x, dy = origin.y + dDebug * dir.y;
+    if (dx >= 0.f && dy >= 0.f && dx < (float)P.gx && dy < (float)P.gy && dDebug < m.d) {
+      m.d = dDebug;
+      m.what = MARCH_DEBUG;
+    }
+  }
+  if (R.solids && (0.f - origin.y) * dir.y > 0.f) {
+    const float dFloor = (0.f - origin.y) / dir.y;
+    if (dFloor < m.d) {
+      m.d = dFloor;
+      m.what = MARCH_FLOOR;
+    }
+  }
+  if (R.solids && P.enable_additional_solids) {
+    float sdf = FLT_MAX, dScene = 0.f;
+    for (int i = 0; i < 100; i++) {
+      sdf = sceneSDF(P, v3add(origin, v3mul(dir, dScene)));
+      if (sdf < 1e-1f || dScene >= m.d) break;
+      dScene = dScene + sdf;
+    }
+    if (sdf < 1e-1f && dScene < m.d) {
+      m.d = dScene;
+      m.what = MARCH_SCENE;
+    }
+    if (R.shadows && (m.what == MARCH_SCENE || m.what == MARCH_FLOOR)) {
+      float3 pos = v3add(origin, v3mul(dir, m.d));
+      if (m.what == MARCH_FLOOR) pos.y = 0.f;
+      m.lt = sceneLight(P, R, pos, sun);
+    }
+  }
+  return m;
+}
+
+// raymarch (src/raymarching.cuh:123-275); returns (color, alpha), the same in the whole group.
+template <int GL, class S>
+__device__ __forceinline__ float4 rayMarch(const S& smp, const dcg_params& P, const dcg_render_params& R, float3 origin,
+                                           float3 dir, float3 sun, const MarchSolid& solid) {
+  using M = MarchGroup<GL>;
   const float ambientInv = 1.f - R.ambient;
   const float floorIllum = fmaxf(0.f, sun.y);
   const float sliceZ = (float)P.gz * .5f;
   const float3 dirInv = make_float3(1.f / dir.x, 1.f / dir.y, 1.f / dir.z);
   const float3 sunInv = make_float3(1.f / sun.x, 1.f / sun.y, 1.f / sun.z);
-  float dCurrent = 0.f;
   float3 color = make_float3(0.f, 0.f, 0.f);
   float alpha = 0.f, illum;
   MarchAux aux;
@@ -160,53 +279,46 @@ __device__ float4 rayMarch(const S& smp, const dcg_params& P, const dcg_render_p
   aux.density = 0.f;
 #pragma unroll
   for (int k = 0; k < 8; k++) aux.cell[k] = 0;
-  float dSolid = FLT_MAX;
-  int what = NONE;
-  if (R.channel != DCG_RENDER_FLUID && (sliceZ - origin.z) * dir.z > 0.f) {
-    const float dDebug = (sliceZ - origin.z) / dir.z;
-    const float dx = origin.x + dDebug * dir.x, dy = origin.y + dDebug * dir.y;
-    if (dx >= 0.f && dy >= 0.f && dx < (float)P.gx && dy < (float)P.gy && dDebug < dSolid) {
-      dSolid = dDebug;
-      what = DEBUG;
-    }
-  }
-  if (R.solids && (0.f - origin.y) * dir.y > 0.f) {
-    const float dFloor = (0.f - origin.y) / dir.y;
-    if (dFloor < dSolid) {
-      dSolid = dFloor;
-      what = FLOOR;
-    }
-  }
-  if (R.solids && P.enable_additional_solids) {
-    float sdf = FLT_MAX, dScene = dCurrent;
-    for (int i = 0; i < 100; i++) {
-      sdf = sceneSDF(P, v3add(origin, v3mul(dir, dScene)));
-      if (sdf < 1e-1f || dScene >= dSolid) break;
-      dScene = dScene + sdf;
-    }
-    if (sdf < 1e-1f && dScene < dSolid) {
-      dSolid = dScene;
-      what = SCENE;
-    }
-  }
+  const float dSolid = solid.d;
+  const int what = solid.what;
   if (R.channel == DCG_RENDER_FLUID) {
     float dNear, dFar;
     if (rayDomain(P, dNear, dFar, origin, dirInv)) {
-      dCurrent = fmaxf(dCurrent, fmaxf(dNear, 10.f));  // Z_NEAR
-      float3 pos = v3add(origin, v3mul(dir, dCurrent));
+      float dCurrent = fmaxf(0.f, fmaxf(dNear, 10.f));  // Z_NEAR
       const float dMax = fminf(dFar, dSolid);
+      const int lane = M::lane();
+      auto next = [&](float d) { return fminf(fmaxf(d * 1.f, d + .5f), dMax); };  // STEP_MULTIPLIER 1
       while (dCurrent < dMax && alpha <= .99f) {
-        const float3 prev = pos;
-        dCurrent = fminf(fmaxf(dCurrent * 1.f, dCurrent + .5f), dMax);  // STEP_MULTIPLIER 1
-        pos = v3add(origin, v3mul(dir, dCurrent));
-        const float3 mid = v3mul(v3add(prev, pos), .5f);
-        smp.sample(P, R.precise, mid, aux);
-        if (aux.density > 1e-6f) {
-          const float sa = densityToAlpha(P, aux.density, v3len(v3sub(pos, prev)));
+        // the next GL steps: lane k goes from the distance after k of them to the one after k + 1
+        float d0 = dCurrent;
+#pragma unroll
+        for (int j = 1; j <= GL; j++) {
+          dCurrent = next(dCurrent);
+          if (j < GL && lane >= j) d0 = dCurrent;
+        }
+        float density = 0.f, sa = 0.f, lt = 1.f;
+        float3 mid = make_float3(0.f, 0.f, 0.f);
+        if (d0 < dMax) {
+          const float3 prev = v3add(origin, v3mul(dir, d0)), pos = v3add(origin, v3mul(dir, next(d0)));
+          mid = v3mul(v3add(prev, pos), .5f);
+          smp.sample(P, R.precise, mid, aux);
+          density = aux.density;
+          if (density > 1e-6f) {
+            sa = densityToAlpha(P, density, v3len(v3sub(pos, prev)));
+            if (R.shadows) lt = sceneLight(P, R, mid, sun);
+          }
+        }
+        // the steps that meet fluid, in order
+        for (uint32_t todo = M::ballot(density > 1e-6f); todo != 0 && alpha <= .99f; todo &= todo - 1) {
+          const int j = __ffs(todo) - 1;
+          const float saj = M::at(sa, j);
           illum = 1.f;
-          if (R.shadows) illum = illum * lightMarch(smp, P, R, mid, aux, sun, sunInv);
+          if (R.shadows) {
+            const float3 mj = make_float3(M::at(mid.x, j), M::at(mid.y, j), M::at(mid.z, j));
+            illum = illum * fluidLight<GL>(smp, P, R, mj, M::at(lt, j), aux, sun, sunInv);
+          }
           illum = R.ambient + illum * ambientInv;
-          marchMix(make_float3(illum * R.smoke_color[0], illum * R.smoke_color[1], illum * R.smoke_color[2]), sa, color,
+          marchMix(make_float3(illum * R.smoke_color[0], illum * R.smoke_color[1], illum * R.smoke_color[2]), saj, color,
                    alpha);
         }
       }
@@ -214,24 +326,24 @@ __device__ float4 rayMarch(const S& smp, const dcg_params& P, const dcg_render_p
   }
   float3 pos = v3add(origin, v3mul(dir, dSolid));
   const float bgAlpha = densityToAlpha(P, 1e-6f, dSolid);
-  if (what == SCENE) {
+  if (what == MARCH_SCENE) {
     const float3 n = sceneNormal(P, pos);
     illum = fmaxf(0.f, n.x * sun.x + n.y * sun.y + n.z * sun.z);
-    if (R.shadows) illum = illum * lightMarch(smp, P, R, pos, aux, sun, sunInv);
+    if (R.shadows) illum = illum * fluidLight<GL>(smp, P, R, pos, solid.lt, aux, sun, sunInv);
     illum = R.ambient + illum * ambientInv;
     marchMix(make_float3(illum * R.scene_color[0], illum * R.scene_color[1], illum * R.scene_color[2]), 1.f - bgAlpha,
              color, alpha);
   }
-  if (what == FLOOR) {
+  if (what == MARCH_FLOOR) {
     pos.y = 0.f;
     illum = floorIllum;
-    if (R.shadows) illum = illum * lightMarch(smp, P, R, pos, aux, sun, sunInv);
+    if (R.shadows) illum = illum * fluidLight<GL>(smp, P, R, pos, solid.lt, aux, sun, sunInv);
     illum = R.ambient + illum * ambientInv;
     illum = illum * (1.f + .1f * fmodf(fabsf(floorf(pos.x / (float)P.gx) + floorf(pos.z / (float)P.gx)), 2.f));
     marchMix(make_float3(illum * R.floor_color[0], illum * R.floor_color[1], illum * R.floor_color[2]), 1.f - bgAlpha,
              color, alpha);
   }
-  if (what == DEBUG) {
+  if (what == MARCH_DEBUG) {
     pos.z = sliceZ;
     smp.sample(P, R.precise, pos, aux);
     if (R.channel == DCG_RENDER_DENSITY) {
@@ -254,28 +366,84 @@ __device__ float4 rayMarch(const S& smp, const dcg_params& P, const dcg_render_p
   return make_float4(color.x, color.y, color.z, alpha);
 }
 
-// k_dcgrid_render / k_uniform_render: per pixel, aa_samples^2 rays averaged.
-template <class S>
-__global__ void __launch_bounds__(256) k_render(S smp, dcg_params P, dcg_render_params R, float4* __restrict__ out) {
-  const int x = blockIdx.x * 16 + (int)(threadIdx.x % 16);
-  const int y = blockIdx.y * 16 + (int)(threadIdx.x / 16);
-  if (x >= R.width || y >= R.height) return;
+// The camera ray of pixel (x, y) offset by (dx, dy).
+__device__ __forceinline__ float3 marchDirection(const dcg_render_params& R, int x, int y, float dx, float dy) {
   const float cx = .5f * (float)R.width, cy = .5f * (float)R.height;
   const float s = R.fov / fmaxf(cx, cy);
+  const float3 view = v3norm(make_float3(((float)x + dx - cx) * s, ((float)y + dy - cy) * s, 1.f));
+  return make_float3(view.x, view.z * R.eye_dir[1] - view.y * R.eye_dir[2], view.y * R.eye_dir[1] + view.z * R.eye_dir[2]);
+}
+__device__ __forceinline__ float3 marchOrigin(const dcg_params& P, const dcg_render_params& R) {
+  return make_float3(R.eye_origin[0] * P.rdx, R.eye_origin[1] * P.rdx, R.eye_origin[2] * P.rdx);
+}
+
+// What every pixel's ray meets behind the fluid, left in the image for k_render (one ray per
+// pixel): d, what and lt in x, y and z.
+static __global__ void __launch_bounds__(256) k_render_solids(dcg_params P, dcg_render_params R, float4* __restrict__ out) {
+  const int x = blockIdx.x * 16 + (int)(threadIdx.x % 16), y = blockIdx.y * 16 + (int)(threadIdx.x / 16);
+  if (x >= R.width || y >= R.height) return;
+  const float3 sun = make_float3(R.sun_dir[0], R.sun_dir[1], R.sun_dir[2]);
+  const MarchSolid m = marchSolid(P, R, marchOrigin(P, R), marchDirection(R, x, y, 0.f, 0.f), sun);
+  out[(size_t)y * R.width + x] = make_float4(m.d, __int_as_float(m.what), m.lt, 0.f);
+}
+
+// k_dcgrid_render / k_uniform_render: per pixel, aa_samples^2 rays averaged. A workgroup takes a
+// tile of T x T pixels with GL lanes per ray. SOLIDS: the pixel's entry of the image holds what its
+// one ray meets behind the fluid (k_render_solids).
+template <int GL, int T, bool SOLIDS, class S>
+__global__ void __launch_bounds__(T* T* GL) k_render(S smp, dcg_params P, dcg_render_params R, float4* __restrict__ out) {
+  const int ray = (int)(threadIdx.x / GL);
+  const int x = blockIdx.x * T + ray % T, y = blockIdx.y * T + ray / T;
+  if (x >= R.width || y >= R.height) return;
   const float step = 1.f / R.aa_samples;
-  const float3 origin = make_float3(R.eye_origin[0] * P.rdx, R.eye_origin[1] * P.rdx, R.eye_origin[2] * P.rdx);
+  const float3 origin = marchOrigin(P, R);
   const float3 sun = make_float3(R.sun_dir[0], R.sun_dir[1], R.sun_dir[2]);
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   for (float dx = 0.f; dx < 1.f; dx = dx + step)
     for (float dy = 0.f; dy < 1.f; dy = dy + step) {
-      const float3 view = v3norm(make_float3(((float)x + dx - cx) * s, ((float)y + dy - cy) * s, 1.f));
-      const float3 dir = make_float3(view.x, view.z * R.eye_dir[1] - view.y * R.eye_dir[2],
-                                     view.y * R.eye_dir[1] + view.z * R.eye_dir[2]);
-      const float4 c = rayMarch(smp, P, R, origin, dir, sun);
+      const float3 dir = marchDirection(R, x, y, dx, dy);
+      MarchSolid solid;
+      if (SOLIDS) {
+        const float4 m = out[(size_t)y * R.width + x];
+        solid = MarchSolid{m.x, __float_as_int(m.y), m.z};
+      } else {
+        solid = marchSolid(P, R, origin, dir, sun);
+      }
+      const float4 c = rayMarch<GL>(smp, P, R, origin, dir, sun, solid);
       acc = make_float4(acc.x + c.x, acc.y + c.y, acc.z + c.z, acc.w + c.w);
     }
+  if (MarchGroup<GL>::lane() != 0) return;
   const float w = step * step;
   out[(size_t)y * R.width + x] = make_float4(acc.x * w, acc.y * w, acc.z * w, acc.w * w);
+}
+
+// The launches of a render. The marched channel takes 16 lanes per ray up to 512 K pixels and 4 above,
+// the debug slices one thread. The ray's fixed cost is paid by every lane, so once the image alone
+// fills the chip fewer lanes win (1920 x 1080, 16 -> 4 lanes: plume 24.1 -> 16.5 ms, dense grid 2.9 ->
+// 1.1 ms, terrain 15.2 -> 11.1 ms; at 512 x 512 16 lanes are the faster, 8.5 -> 4.4 ms on the plume).
+// A solid scene's sphere traces (up to 200 scene distances a ray, each a 5-octave noise with a
+// terrain) cannot be shared by a ray's lanes: a pass of its own takes them a thread per ray, and
+// leaves its results in the image, which holds them for one ray per pixel; with several the whole
+// march runs a thread per ray (a trace by 16 lanes alike takes 16 times the instructions: a terrain
+// image of 1024 x 768 took 17.8 ms with the traces in the march's workgroups, 4.4 ms this way).
+template <class S>
+void launchRender(const S& smp, const dcg_params& P, const dcg_render_params& R, float4* out, hipStream_t stream) {
+  auto grid = [&](int t) { return dim3((unsigned)((R.width + t - 1) / t), (unsigned)((R.height + t - 1) / t)); };
+  const bool scene = R.solids && P.enable_additional_solids;
+  const bool wide = (size_t)R.width * R.height <= (size_t)512 * 1024;
+  if (R.channel != DCG_RENDER_FLUID || (scene && R.aa_samples > 1.f)) {
+    k_render<1, 16, false><<<grid(16), 256, 0, stream>>>(smp, P, R, out);
+  } else if (scene) {
+    k_render_solids<<<grid(16), 256, 0, stream>>>(P, R, out);
+    if (wide)
+      k_render<16, 4, true><<<grid(4), 256, 0, stream>>>(smp, P, R, out);
+    else
+      k_render<4, 8, true><<<grid(8), 256, 0, stream>>>(smp, P, R, out);
+  } else if (wide) {
+    k_render<16, 4, false><<<grid(4), 256, 0, stream>>>(smp, P, R, out);
+  } else {
+    k_render<4, 8, false><<<grid(8), 256, 0, stream>>>(smp, P, R, out);
+  }
 }
 
 }  // namespace dcg

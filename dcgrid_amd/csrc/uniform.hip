@@ -724,9 +724,8 @@ struct UniformSim : SimBase {
     }
   }
   int render(const dcg_render_params& r, float* rgba) override {
-    const dim3 grid((unsigned)((r.width + 15) / 16), (unsigned)((r.height + 15) / 16));
     UMarchSampler smp{g};
-    DCG_LAUNCH(DCG_K_OTHER, "k_render", (k_render<<<grid, 256, 0, stream>>>(smp, P, r, (float4*)rgba)));
+    DCG_LAUNCH(DCG_K_OTHER, "k_render", (launchRender(smp, P, r, (float4*)rgba, stream)));
     return DCG_OK;
   }
 

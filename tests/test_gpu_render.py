@@ -110,3 +110,27 @@ def test_device_pointer_and_checks():
         g.render(bad)
     g.close()
     c.close()
+
+
+@pytest.mark.parametrize("name,size", [("cfg1_64", (1, 1)), ("cfg1_64", (5, 3)), ("ref64_bw4_solids", (17, 9)),
+                                       ("cfg0_32_solids", (4, 4)), ("cfg1_64", (1025, 512)),
+                                       ("cfg0_32_solids", (1025, 512))])
+def test_render_lanes_per_ray(name, size):
+    """The marched channel at the edges of its launch shapes: partial tiles (an image smaller than a
+    tile, one past it), and one pixel row past the 512 K pixels from which 4 lanes take a ray instead
+    of 16. The small images equal the oracle's; the large one's inner rows equal those of an image
+    two rows lower, which takes 16 lanes."""
+    g, c = pair(name)
+    r = g.default_render_params()
+    r.width, r.height = size
+    a = g.render(r)
+    if size[0] * size[1] <= 1024:
+        assert same(a, c.render(r)), (name, size)
+    else:  # the same rays from a narrower image: the pixel pitch follows the larger side
+        half = r.copy()
+        half.height = size[1] - 2
+        b = g.render(half)
+        assert size[0] * size[1] > 512 * 1024 >= half.width * half.height
+        assert same(a[1:-1], b), (name, size)
+    g.close()
+    c.close()
