@@ -235,6 +235,26 @@ __device__ __forceinline__ float sourceTemperature(const dcg_params& P, int x, i
 __device__ __forceinline__ float3 f3mul(float3 a, float s) { return make_float3(a.x * s, a.y * s, a.z * s); }
 __device__ __forceinline__ float3 f3add(float3 a, float3 b) { return make_float3(a.x + b.x, a.y + b.y, a.z + b.z); }
 
+// x / 6 correctly rounded, as the division gives it, in 4 operations instead of the division's 11
+// (one of them a quarter-rate reciprocal): the quotient by the rounded reciprocal, its exact
+// residual by FMA and one correction (Brisebarre, Muller, Raina, "Accelerating correctly rounded
+// floating-point division when the divisor is known in advance", IEEE Trans. Computers 2004);
+// v_div_fixup settles zeros, infinities and NaN. Equal to x / 6.f on all 2^32 floats except
+// where the quotient is subnormal (ties of the last place): sixthUnsure() of the result tells, and
+// the caller divides instead.
+__device__ __forceinline__ float sixthFast(float x) {
+  constexpr float r = 1.f / 6.f;
+  const float q = x * r;
+  const float e = __builtin_fmaf(-6.f, q, x);
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(e, r, q), 6.f, x);
+}
+__device__ __forceinline__ bool sixthUnsure(float q) { return __builtin_amdgcn_classf(q, 0x010 | 0x080); }
+__device__ __forceinline__ float sixth(float x) {
+  float q = sixthFast(x);
+  if (sixthUnsure(q)) q = x / 6.f;
+  return q;
+}
+
 // XCD-aware remap of a linear workgroup id: consecutive ids are dispatched round-robin over the
 // 8 XCDs of MI355X; this maps them so each XCD works on a contiguous range (shared L2 reuse).
 __device__ __forceinline__ uint32_t xcdRemap(uint32_t id, uint32_t n) {

@@ -219,9 +219,10 @@ __global__ void __launch_bounds__(256) k_u_advect_density(dcg_params P, UGrid g)
   g.tden[i] = q;
 }
 
-// k_uniform_calc_divergence, uniformgrid_fluid.cu:107-132
+// k_uniform_calc_divergence, uniformgrid_fluid.cu:107-132. zero: clear both pressure arrays (not where
+// the sweeps that follow write every cell of both without reading them).
 template <bool FLUIDITY>
-__global__ void __launch_bounds__(256) k_u_divergence(dcg_params P, UGrid g) {
+__global__ void __launch_bounds__(256) k_u_divergence(dcg_params P, UGrid g, int zero) {
   const size_t n = (size_t)g.gx * g.gy * g.gz;
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
@@ -231,8 +232,10 @@ __global__ void __launch_bounds__(256) k_u_divergence(dcg_params P, UGrid g) {
   const size_t il = x > 0 ? i - 1 : i, ir = x < g.gx - 1 ? i + 1 : i;
   const size_t id = y > 0 ? i - g.gx : i, iu = y < g.gy - 1 ? i + g.gx : i;
   const size_t ib = z > 0 ? i - pl : i, iF = z < g.gz - 1 ? i + pl : i;
-  g.pre[i] = 0.f;
-  g.tpre[i] = 0.f;
+  if (zero) {
+    g.pre[i] = 0.f;
+    g.tpre[i] = 0.f;
+  }
   const float wl = FLUIDITY ? g.flu[il] : 1.f, wr = FLUIDITY ? g.flu[ir] : 1.f;
   const float wd = FLUIDITY ? g.flu[id] : 1.f, wu = FLUIDITY ? g.flu[iu] : 1.f;
   const float wb = FLUIDITY ? g.flu[ib] : 1.f, wf = FLUIDITY ? g.flu[iF] : 1.f;
@@ -314,6 +317,122 @@ __global__ void __launch_bounds__(256) k_u_prolongate(float* __restrict__ pre, U
   uProlongCell(pre, L, Lp, i);
 }
 
+// K Jacobi half-sweeps of a level in one launch, bit for bit the values of K launches of k_u_jacobi.
+// A single half-sweep of a grid that fits the caches is a launch (about 2.5 us) and a round trip to the
+// other XCDs' results for 0.2 us of work, and of a large one 12 B of HBM per cell: several sweeps of a
+// tile in registers share both. Measured (MI355X, k_u_jacobi -> k_u_sweeps, whole projections): 64^3 with
+// 100 sweeps 283 -> 161 us, 128^3 with 40 sweeps 336 -> 233 us, 320 x 256 x 384 with 10 sweeps 1507 ->
+// 940 us, multilevel 857 -> 657 us.
+// A workgroup takes 64 x TY x TZ cells grown by K cells in y and z and, on a level wider than a
+// wavefront, in x. A wavefront is a row of 64 cells along x and keeps the rows of one y in
+// registers: x neighbours come by DPP, z neighbours from the same thread, y neighbours from LDS.
+// Every sweep the region of valid rows shrinks by one; the clamped neighbours of the domain's border
+// cells are the cells themselves, so no halo is needed there. The first sweep's input: zero
+// (inMode 0), an array (1) or the prolonged pressure of the coarser level (2). The last sweep is
+// written to `out`, the one before it to `outPrev` where that is given; neither may be the input.
+enum : int { U_IN_ZERO = 0, U_IN_ARRAY = 1, U_IN_PROLONG = 2 };
+template <int K, int TY, int TZ>
+__global__ void __launch_bounds__((TY + 2 * K) * 64) k_u_sweeps(const float* __restrict__ in, int inMode,
+                                                                const float* __restrict__ div, float* __restrict__ out,
+                                                                float* __restrict__ outPrev, int w, int h, int d,
+                                                                int nx, int ny, float alpha) {
+  constexpr int NW = TY + 2 * K, ZR = TZ + 2 * K;
+  __shared__ float rows[NW][ZR][64];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // tiles in x, y, z order, a contiguous range of them per XCD
+  const uint32_t id = xcdRemap(blockIdx.x, gridDim.x), ty = id / (uint32_t)nx;
+  const int tx = (int)(id - ty * (uint32_t)nx), tz = (int)(ty / (uint32_t)ny);
+  const int x = tx * (64 - 2 * K) + lane, y = ((int)ty - tz * ny) * TY - K + wv, z0 = tz * TZ - K;
+  const int xc = min(x, w - 1), yc = clampi(y, 0, h - 1);
+  float p[ZR], ad[ZR];
+  auto rowOf = [&](int k) {
+    return ((uint32_t)clampi(z0 + k, 0, d - 1) * (uint32_t)h + (uint32_t)yc) * (uint32_t)w + (uint32_t)xc;
+  };
+#pragma unroll
+  for (int k = 0; k < ZR; k++) ad[k] = div[rowOf(k)];
+  if (inMode == U_IN_PROLONG) {
+    // uProlongCell: per coarser plane the four values of the cell's (x, y) stencil, shared by the
+    // rows that read the plane
+    const int cw = w / 2, ch = h / 2, cd = d / 2;
+    const int sx = (xc == 0 || xc == w - 1) ? 0 : 2 * (xc & 1) - 1, sy = (yc == 0 || yc == h - 1) ? 0 : 2 * (yc & 1) - 1;
+    const uint32_t c00 = (uint32_t)(yc >> 1) * (uint32_t)cw + (uint32_t)(xc >> 1), c01 = c00 + sx;
+    const uint32_t c10 = (uint32_t)((yc >> 1) + sy) * (uint32_t)cw + (uint32_t)(xc >> 1), c11 = c10 + sx;
+    constexpr int PAR = K & 1, NP = (ZR + PAR + 1) / 2 + 2;  // z0 has K's parity (TZ is even)
+    static_assert(TZ % 2 == 0, "the rows' parity is a constant");
+    const int cz0 = ((z0 - PAR) >> 1) - 1;  // coarser plane of entry 0
+    float q[NP][4];
+#pragma unroll
+    for (int c = 0; c < NP; c++) {
+      const float* pl = in + (uint32_t)clampi(cz0 + c, 0, cd - 1) * (uint32_t)cw * (uint32_t)ch;
+      q[c][0] = pl[c00];
+      q[c][1] = pl[c01];
+      q[c][2] = pl[c10];
+      q[c][3] = pl[c11];
+    }
+#pragma unroll
+    for (int k = 0; k < ZR; k++) {
+      const int z = z0 + k, c = (k + PAR) / 2 + 1, o = (k + PAR) % 2 ? c + 1 : c - 1;
+      const bool flat = z <= 0 || z >= d - 1;  // no z neighbour at the border planes
+      float n[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) n[j] = flat ? q[c][j] : q[o][j];
+      p[k] = (27.f * q[c][0] + 9.f * (q[c][1] + q[c][2] + n[0]) + 3.f * (q[c][3] + n[1] + n[2]) + n[3]) / 64.f;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < ZR; k++) p[k] = inMode == U_IN_ARRAY ? in[rowOf(k)] : 0.f;
+  }
+#pragma unroll
+  for (int k = 0; k < ZR; k++) ad[k] = alpha * ad[k];
+  const bool right = x >= w - 1;  // the last cell's right neighbour is itself (its left one: lane 0 keeps its own)
+  const int yd = y <= 0 || wv == 0 ? wv : wv - 1, yu = y >= h - 1 || wv == NW - 1 ? wv : wv + 1;
+  const bool mine = wv >= K && wv < K + TY && y < h && x < w && (tx == 0 || lane >= K) && (lane < 64 - K || tx == nx - 1);
+  auto store = [&](float* __restrict__ to) {
+    if (!mine) return;
+#pragma unroll
+    for (int k = K; k < K + TZ; k++)
+      if (z0 + k < d) to[((uint32_t)(z0 + k) * (uint32_t)h + (uint32_t)y) * (uint32_t)w + (uint32_t)x] = p[k];
+  };
+#pragma unroll
+  for (int s = 1; s <= K; s++) {
+    if (s > 1) __syncthreads();  // the last sweep's rows are no longer read
+    if (wv >= s - 1 && wv <= NW - s) {
+#pragma unroll
+      for (int k = s; k < ZR - s; k++) rows[wv][k][lane] = p[k];
+    }
+    __syncthreads();
+    if (wv >= s && wv < NW - s) {
+      float last = p[s - 1];
+      float v[ZR];
+#pragma unroll
+      for (int k = s; k < ZR - s; k++) {
+        const float c = p[k];
+        // wave_shr:1, wave_shl:1
+        const float l = __int_as_float(
+            __builtin_amdgcn_update_dpp(__float_as_int(c), __float_as_int(c), 0x138, 0xF, 0xF, false));
+        float r = __int_as_float(
+            __builtin_amdgcn_update_dpp(__float_as_int(c), __float_as_int(c), 0x130, 0xF, 0xF, false));
+        r = right ? c : r;
+        const float b = z0 + k <= 0 ? c : last, f = z0 + k >= d - 1 ? c : p[k + 1];
+        v[k] = l + r + rows[yd][k][lane] + rows[yu][k][lane] + b + f - ad[k];
+        last = c;
+      }
+      bool unsure = false;
+#pragma unroll
+      for (int k = s; k < ZR - s; k++) {
+        p[k] = sixthFast(v[k]);
+        unsure |= sixthUnsure(p[k]);
+      }
+      if (__ballot(unsure) != 0) {
+#pragma unroll
+        for (int k = s; k < ZR - s; k++) p[k] = v[k] / 6.f;
+      }
+    }
+    if (s == K - 1 && outPrev) store(outPrev);
+  }
+  store(out);
+}
+
 // The levels of the pyramid small enough for one workgroup (<= kCoarseCells cells each),
 // finest first: their part of project() (restriction into them, the top level's sweeps, and
 // prolongation and sweeps back down to the first of them) in one launch. Their pressure,
@@ -327,7 +446,7 @@ constexpr int kCoarseLds = 4096 + 512 + 64 + 8 + 1 + 1;  // >= sum of a geometri
 struct ULevels {
   UDims d[DCG_MAX_LEVELS];
 };
-__device__ __forceinline__ size_t ucells(const UDims& D) { return (size_t)D.w * D.h * D.d; }
+__host__ __device__ __forceinline__ size_t ucells(const UDims& D) { return (size_t)D.w * D.h * D.d; }
 // Dimensions of levels Ls.. with offsets relative to level Ls (their LDS layout).
 __device__ __forceinline__ void coarseLocal(const ULevels& D, int L, int Ls, ULevels& S, size_t& total) {
   total = 0;
@@ -358,7 +477,7 @@ __global__ void __launch_bounds__(1024) k_u_coarse(UGrid g, ULevels D, int L, in
   }
   auto sweeps = [&](int l, int pairs) {
     const int scale = 1 << l;
-    const float alpha = dx * dx * (float)scale * (float)scale;  // as jacobiPairs
+    const float alpha = dx * dx * (float)scale * (float)scale;  // dx*dx*scale*scale, uniformgrid_fluid.cu:171
     for (int p = 0; p < pairs; p++) {
       for (size_t i = threadIdx.x; i < ucells(S.d[l]); i += blockDim.x) uJacobiCell(sp, st, sd, S.d[l], alpha, i);
       __syncthreads();
@@ -575,26 +694,66 @@ struct UniformSim : SimBase {
     if (src) std::swap(g.tem, g.ttem);
     return DCG_OK;
   }
-  int divergence() {
+  int divergence(bool zero) {
+    const int z = zero ? 1 : 0;
     if (fluidityOn())
-      DCG_LAUNCH(DCG_K_DIVERGENCE, "k_u_divergence", (k_u_divergence<true><<<nblk(N), 256, 0, stream>>>(P, g)));
+      DCG_LAUNCH(DCG_K_DIVERGENCE, "k_u_divergence", (k_u_divergence<true><<<nblk(N), 256, 0, stream>>>(P, g, z)));
     else
-      DCG_LAUNCH(DCG_K_DIVERGENCE, "k_u_divergence", (k_u_divergence<false><<<nblk(N), 256, 0, stream>>>(P, g)));
+      DCG_LAUNCH(DCG_K_DIVERGENCE, "k_u_divergence", (k_u_divergence<false><<<nblk(N), 256, 0, stream>>>(P, g, z)));
     return DCG_OK;
   }
-  int jacobiPairs(int level, int pairs) {
+  // The 2 `pairs` half-sweeps of a level from a first input that is not the pressure array: zero, or
+  // the prolonged pressure of the coarser level. Chunks of at most 4 sweeps a launch pass their
+  // results through scratch (the advected velocity's second buffer, free between the advections);
+  // the last one writes the last sweep to the pressure and the one before to t_pressure.
+  // Tiles: 4 x 4 in (y, z) while these are at most two per CU, so that every CU has one (64^3, 100
+  // sweeps: 4 x 4 161 us, 8 x 8 232 us); larger ones beyond, where the halo's redundant rows cost more
+  // (128^3, 40 sweeps: 391 against 233 us; 96 x 100 x 104: 215 against 158 us). Five sweeps a launch
+  // measured slower than four (128^3: 316 us), three about equal. Two sweeps (a level of the
+  // multilevel schedule) take 8 x 8, and 12 x 12 from 1024 tiles (320 x 256 x 384 projection: 674
+  // against 660 us).
+  static constexpr int kSweepsPerLaunch = 4;
+  static int sweepColumns(int w, int k) { return w <= 64 ? 1 : (w - 64 + (64 - 2 * k) - 1) / (64 - 2 * k) + 1; }
+  static size_t sweepTiles(const UDims& D, int k, int ty, int tz) {
+    return (size_t)sweepColumns(D.w, k) * (size_t)((D.h + ty - 1) / ty) * (size_t)((D.d + tz - 1) / tz);
+  }
+  template <int K, int TY, int TZ>
+  void sweepLaunch(const UDims& D, const float* in, int mode, float* out, float* outPrev, float alpha) {
+    k_u_sweeps<K, TY, TZ><<<(unsigned)sweepTiles(D, K, TY, TZ), (TY + 2 * K) * 64, 0, stream>>>(
+        in, mode, g.div + D.off, out, outPrev, D.w, D.h, D.d, sweepColumns(D.w, K), (D.h + TY - 1) / TY, alpha);
+  }
+  int sweeps(int level, int pairs, int mode) {
     const UDims& D = dims[level];
-    const size_t n = (size_t)D.w * D.h * D.d;
+    const size_t n = ucells(D);
     const int scale = 1 << level;
-    // alpha = dx*dx*scale*scale, uniformgrid_fluid.cu:171
-    const float alpha = P.dx * P.dx * (float)scale * (float)scale;
-    if (pairs <= 0) return DCG_OK;
-    Pending batch;  // the run of back-to-back sweeps is timed as one batch
+    const float alpha = P.dx * P.dx * (float)scale * (float)scale;  // dx*dx*scale*scale, uniformgrid_fluid.cu:171
+    const float* in = mode == U_IN_PROLONG ? g.pre + dims[level + 1].off : nullptr;
+    float* scratch[2] = {(float*)g.tvel, (float*)g.tvel + n};
+    int left = 2 * pairs, chunks = (left + kSweepsPerLaunch - 1) / kSweepsPerLaunch;
+    Pending batch;  // the run of launches is timed as one batch of half-sweeps
     DCG_TRY(beginTimed(DCG_K_JACOBI, &batch));
     batchK = DCG_K_JACOBI;
-    for (int i = 0; i < pairs; i++) {
-      DCG_LAUNCH(DCG_K_JACOBI, "k_u_jacobi", (k_u_jacobi<<<nblk(n), 256, 0, stream>>>(g.pre, g.tpre, g.div, D, alpha)));
-      DCG_LAUNCH(DCG_K_JACOBI, "k_u_jacobi", (k_u_jacobi<<<nblk(n), 256, 0, stream>>>(g.tpre, g.pre, g.div, D, alpha)));
+    for (int c = 0; chunks > 0; c++, chunks--) {
+      const int k = (left + chunks - 1) / chunks;
+      left -= k;
+      float* out = chunks == 1 ? g.pre + D.off : scratch[c & 1];
+      float* outPrev = chunks == 1 ? g.tpre + D.off : nullptr;
+      const size_t small = sweepTiles(D, k, 4, 4), wide = sweepTiles(D, k, 12, 12);
+      if (small <= 512) {
+        if (k == 2) sweepLaunch<2, 4, 4>(D, in, mode, out, outPrev, alpha);
+        else if (k == 3) sweepLaunch<3, 4, 4>(D, in, mode, out, outPrev, alpha);
+        else sweepLaunch<4, 4, 4>(D, in, mode, out, outPrev, alpha);
+      } else if (k == 2) {
+        if (wide >= 1024) sweepLaunch<2, 12, 12>(D, in, mode, out, outPrev, alpha);
+        else sweepLaunch<2, 8, 8>(D, in, mode, out, outPrev, alpha);
+      } else if (k == 3) {
+        sweepLaunch<3, 10, 10>(D, in, mode, out, outPrev, alpha);
+      } else {
+        sweepLaunch<4, 8, 8>(D, in, mode, out, outPrev, alpha);
+      }
+      DCG_TRY(checkLaunch("k_u_sweeps"));
+      in = out;
+      mode = U_IN_ARRAY;
     }
     batchK = -1;
     return endTimed(DCG_K_JACOBI, &batch, 2 * pairs);
@@ -657,8 +816,10 @@ struct UniformSim : SimBase {
   // project(), fluid_simulation_uniform.cu:96-124; the levels from coarseStart() up run in one
   // workgroup (k_u_coarse), the others level by level.
   int project() override {
-    DCG_TRY(divergence());
     const int Ls = coarseStart();
+    // level 0 is swept by sweeps(), which writes all of its pressure and t_pressure
+    const bool swept = Ls > 0 && (L > 1 ? P.project_level_pairs : P.project_top_pairs) > 0;
+    DCG_TRY(divergence(!swept));
     for (int l = 1; l < L && l <= Ls; l++) {
       const UDims& D = dims[l];
       DCG_LAUNCH(DCG_K_RESTRICT, "k_u_restrict", (k_u_restrict<<<nblk((size_t)D.w * D.h * D.d), 256, 0, stream>>>(g, D, dims[l - 1])));
@@ -666,20 +827,23 @@ struct UniformSim : SimBase {
     if (Ls < L) {
       DCG_LAUNCH(DCG_K_JACOBI, "k_u_coarse",
                  (k_u_coarse<<<1, 1024, 0, stream>>>(g, levels(), L, Ls, P.project_top_pairs, P.project_level_pairs, P.dx)));
-    } else {
-      DCG_TRY(jacobiPairs(L - 1, P.project_top_pairs));
+    } else if (P.project_top_pairs > 0) {
+      DCG_TRY(sweeps(L - 1, P.project_top_pairs, U_IN_ZERO));
     }
     for (int l = std::min(Ls, L - 1) - 1; l >= 0; l--) {
       const UDims& D = dims[l];
+      if (P.project_level_pairs > 0) {
+        DCG_TRY(sweeps(l, P.project_level_pairs, U_IN_PROLONG));
+        continue;
+      }
       DCG_LAUNCH(DCG_K_PROLONGATE, "k_u_prolongate", (k_u_prolongate<<<nblk((size_t)D.w * D.h * D.d), 256, 0, stream>>>(g.pre, D, dims[l + 1])));
-      DCG_TRY(jacobiPairs(l, P.project_level_pairs));
     }
     return applyPressure();
   }
   // projectLocal(), fluid_simulation_uniform.cu:126-135
   int projectLocal() override {
-    DCG_TRY(divergence());
-    DCG_TRY(jacobiPairs(0, P.project_local_pairs));
+    DCG_TRY(divergence(P.project_local_pairs <= 0));
+    if (P.project_local_pairs > 0) DCG_TRY(sweeps(0, P.project_local_pairs, U_IN_ZERO));
     return applyPressure();
   }
   // debugStats(), fluid_simulation_uniform.cu:160-175
@@ -982,7 +1146,7 @@ struct UniformSim : SimBase {
     const bool perLevel = stage == DCG_STAGE_JACOBI || stage == DCG_STAGE_JACOBI_INV || stage == DCG_STAGE_PROLONGATE;
     if (perLevel && (arg < 0 || arg >= L || (stage == DCG_STAGE_PROLONGATE && arg >= L - 1)))
       return fail(DCG_E_ARG, "level out of range");
-    if (stage == DCG_STAGE_DIVERGENCE) return divergence();
+    if (stage == DCG_STAGE_DIVERGENCE) return divergence(true);
     if (stage == DCG_STAGE_RESTRICT) {
       for (int l = 1; l < L; l++) {
         const UDims& D = dims[l];
