@@ -4,7 +4,9 @@
 // move limits and selection results stay in device control words, and kernels whose work depends
 // on them are launched over the static per-level capacity and exit early.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
+#include <map>
 #include <type_traits>
 
 #include <hip/hip_ext.h>
@@ -12,6 +14,7 @@
 #include "dcg_internal.hpp"
 #include "dcgrid_fluid.hpp"
 #include "dcgrid_solve.hpp"
+#include "dcgrid_direct.hpp"
 #include "dcgrid_topo.hpp"
 #include "dcgrid_adjoint.hpp"
 #include "render.hpp"
@@ -713,6 +716,120 @@ struct DCGridSim : SimBase {
     DCG_TRY(fill32(coarseTags, 0u, (size_t)L));
     return DCG_OK;
   }
+  // ---- direct solve of the dense levels (dcgrid_direct.hpp)
+  // Transform matrices per axis length, in FP64 and FP32, laid out once.
+  std::map<int, DctAxis<double>> dctD;
+  std::map<int, DctAxis<float>> dctF;
+  int axisCells(int l, int axis) const { return BW * (axis == 0 ? g.rx[l] : axis == 1 ? g.ry[l] : g.rz[l]); }
+  // A dense level (all of its blocks allocated at creation: no ghosts, Neumann walls) whose axes fit
+  // the transform's LDS tile, on FP32 fields. 16-bit fields keep the V-cycles: the two solutions agree
+  // within the tolerance (5e-9), but where that crosses a rounding boundary of the stored pressure or
+  // velocity a value moves by its last place (2^-8), and later steps carry that on; eight steps of
+  // configuration 2 in BF16 part by 8.5e-5 in the rendered image, FP32 fields by 1e-8 a projection. So
+  // runs on 16-bit fields stay what they were, bit for bit.
+  bool directLevel(int l) const {
+    if (!std::is_same<SF, float>::value || l < S) return false;
+    for (int a = 0; a < 3; a++)
+      if (axisCells(l, a) > kDctMaxAxis) return false;
+    return true;
+  }
+  template <class T>
+  int dctAxis(int n, std::map<int, DctAxis<T>>& axes) {
+    if (axes.count(n)) return DCG_OK;
+    DctAxis<T> ax{};
+    ax.n = n;
+    ax.nh = n / 2;
+    ax.np = (ax.nh + 15) / 16 * 16;
+    const size_t m = (size_t)ax.np * ax.np;
+    std::vector<T> h(4 * m + n, (T)0);
+    const double pi = 3.14159265358979323846;
+    std::vector<double> cosine(4 * n);  // of pi m / 2 n, one period
+    for (int m2 = 0; m2 < 4 * n; m2++) cosine[m2] = std::cos(pi * m2 / (2.0 * n));
+    for (int par = 0; par < 2; par++)
+      for (int k = 0; k < ax.nh; k++)
+        for (int i = 0; i < ax.nh; i++) {
+          const int f = 2 * k + par;  // (f (2 i + 1) stays below 2 n^2)
+          const T v = (T)(cosine[f * (2 * i + 1) % (4 * n)] * std::sqrt((f == 0 ? 1.0 : 2.0) / n));
+          h[par * m + (size_t)k * ax.np + i] = v;
+          h[(2 + par) * m + (size_t)i * ax.np + k] = v;
+        }
+    for (int r = 0; r < n; r++) {
+      const int f = r < ax.nh ? 2 * r : 2 * (r - ax.nh) + 1;
+      const double s = std::sin(pi * f / (2.0 * n));
+      h[4 * m + r] = (T)(4.0 * s * s);
+    }
+    T* d = nullptr;
+    DCG_TRY(alloc(&d, h.size()));
+    DCG_HIP(hipMemcpyAsync(d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, stream));
+    DCG_TRY(sync());
+    for (int par = 0; par < 2; par++) {
+      ax.fwd[par] = d + par * m;
+      ax.inv[par] = d + (2 + par) * m;
+    }
+    ax.lam = d + 4 * m;
+    axes[n] = ax;
+    return DCG_OK;
+  }
+  std::map<int, DctAxis<double>>& dctAxes(double) { return dctD; }
+  std::map<int, DctAxis<float>>& dctAxes(float) { return dctF; }
+  template <class T>
+  int dctSetup() {
+    for (int l = S; l < L; l++)
+      if (directLevel(l))
+        for (int a = 0; a < 3; a++) DCG_TRY(dctAxis<T>(axisCells(l, a), dctAxes(T())));
+    return DCG_OK;
+  }
+  template <class T, int NC, int PASS>
+  int dctPass(const DctArgs<T>& a, unsigned tiles) {
+    const size_t lds = dctLds<T, NC>(a.ax.np);
+    if (lds > 64 * 1024)
+      DCG_HIP(hipFuncSetAttribute((const void*)k_dct<BW, T, NC, PASS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    DCG_LAUNCH(DCG_K_SOLVE, "k_dct", (k_dct<BW, T, NC, PASS><<<tiles, kDctThreads, lds, stream>>>(a)));
+    return DCG_OK;
+  }
+  // One pass over the level: tiles of 64 lines while they fill the chip and fit the LDS (an axis of 256
+  // in FP64), else of 32, and of 16 beyond 512 entries.
+  template <class T, int PASS>
+  int dctLaunch(int l, const T* in, T* out, const SolveCtl* ctl) {
+    auto& axes = dctAxes(T());
+    DctArgs<T> a{};
+    a.nx = axisCells(l, 0);
+    a.ny = axisCells(l, 1);
+    a.nz = axisCells(l, 2);
+    a.rx = g.rx[l];
+    a.ry = g.ry[l];
+    a.rz = g.rz[l];
+    a.ax = axes[PASS == DCT_X_BOTH ? a.nx : (PASS == DCT_Y_FWD || PASS == DCT_Y_INV) ? a.ny : a.nz];
+    a.lamY = axes[a.ny].lam;
+    a.lamZ = axes[a.nz].lam;
+    a.in = in;
+    a.out = out;
+    a.cell0 = offs[l] * G::BV;
+    a.h2 = (T)levelH2(l);
+    a.ctl = ctl;
+    auto tiles = [&](int nc) {
+      if (PASS == DCT_X_BOTH) return blocksFor((size_t)a.ny * a.nz, nc);
+      if (PASS == DCT_Y_FWD || PASS == DCT_Y_INV) return (unsigned)a.rx * blocksFor(a.nz, nc / BW);
+      return blocksFor((size_t)a.nx * a.ny, nc);
+    };
+    if (a.ax.n > 512) return dctPass<T, 16, PASS>(a, tiles(16));
+    if (a.ax.n > 256 || tiles(64) < 256) return dctPass<T, 32, PASS>(a, tiles(32));
+    return dctPass<T, 64, PASS>(a, tiles(64));
+  }
+  // e of dense level l from rho. The level's slices of `s1` (the iterate buffer the next residual
+  // writes) and of rho (which it recomputes) hold the transforms' intermediate values.
+  template <class T>
+  int directSolve(int l, T* s1, const SolveCtl* ctl) {
+    T* rho = (T*)rhoBuf;
+    T* e = (T*)eBuf;
+    T* a1 = s1 + (size_t)offs[l] * G::BV;
+    T* a2 = rho + (size_t)offs[l] * G::BV;
+    DCG_TRY((dctLaunch<T, DCT_Z_FWD>(l, rho, a1, ctl)));
+    DCG_TRY((dctLaunch<T, DCT_Y_FWD>(l, a1, a2, ctl)));
+    DCG_TRY((dctLaunch<T, DCT_X_BOTH>(l, a2, a2, ctl)));
+    DCG_TRY((dctLaunch<T, DCT_Y_INV>(l, a2, a1, ctl)));
+    return dctLaunch<T, DCT_Z_INV>(l, a1, e, ctl);
+  }
   // Ghost factor of a Dirichlet face on the grid m levels coarser than the solved level: the
   // finest grid puts the zero half a fine cell beyond the region's face, i.e. at
   // d = (1/2 + 2^-(m+1)) coarse cells from the boundary cell's centre; the linear ghost through
@@ -925,15 +1042,19 @@ struct DCGridSim : SimBase {
     const double tol = P.solve_tol > 0 ? (double)P.solve_tol : 1e-8;
     const int maxCycles = P.solve_max_cycles > 0 ? P.solve_max_cycles : 50;
     DCG_TRY((residualLaunch<TX, T>(l, true, xc, xc, ctl)));
+    const bool direct = directLevel(l);
     int issued = 0;
-    int n = predCycles[l] > 0 ? predCycles[l] : 6;
+    int n = predCycles[l] > 0 ? predCycles[l] : direct ? 1 : 6;
     SolveCtl h{};
     for (;;) {
       for (int i = 0; i < n && issued <= maxCycles; i++, issued++) {
-        DCG_TRY(vcycle<T>(l, ctl));
         // cycle i+1 reads the iterate of cycle i and writes the other buffer
         TX* xin = issued % 2 == 0 ? xc : x2;
         TX* xout = issued % 2 == 0 ? x2 : xc;
+        if (direct)
+          DCG_TRY(directSolve<T>(l, (T*)xout, ctl));
+        else
+          DCG_TRY(vcycle<T>(l, ctl));
         DCG_TRY((residualLaunch<TX, T>(l, false, xin, xout, ctl)));
       }
       DCG_TRY(sync());  // the decide kernel mirrored the control block into pinned host memory
@@ -960,6 +1081,12 @@ struct DCGridSim : SimBase {
   int solveAll(bool warm) {
     TX* xc = (TX*)xBuf[0];
     for (int l = L - 1; l >= 0; l--) {
+      // a dense level solved directly in FP64 needs no guess
+      if (std::is_same<TX, double>::value && directLevel(l)) {
+        if (!warm) DCG_LAUNCH(DCG_K_SOLVE, "k_sv_zero", (k_sv_zero<BW, TX><<<cellGrid(l), 256, 0, stream>>>(g, l, xc)));
+        DCG_TRY((solveLevel<double, double>(l)));
+        continue;
+      }
       if (l == L - 1) {
         if (!warm) DCG_LAUNCH(DCG_K_SOLVE, "k_sv_zero", (k_sv_zero<BW, TX><<<cellGrid(l), 256, 0, stream>>>(g, l, xc)));
       } else {
@@ -979,6 +1106,9 @@ struct DCGridSim : SimBase {
       DCG_LAUNCH(DCG_K_SOLVE, "k_sv_warm", (k_sv_warm<BW, TX><<<n, 256, 0, stream>>>(g, (TX*)xBuf[0])));
     }
     DCG_TRY(divergence());
+    int cyc = L;  // the levels below `cyc` run V-cycles
+    while (cyc > 0 && directLevel(cyc - 1)) cyc--;
+    if (cyc == 0) return solveAll<TX, T>(warm);
     for (int l = 0; l < L; l++)
       DCG_LAUNCH(DCG_K_SOLVE, "k_sv_reach",
                  (k_sv_reach<BW><<<slotGrid<BW>(maxL[l]), G::WG, 0, stream>>>(g, l, reachBuf, breachBuf)));
@@ -988,7 +1118,7 @@ struct DCGridSim : SimBase {
     {
       unsigned n = blocksFor(maxL[0], 256);
       for (int l = 1; l < L; l++) n = std::max(n, blocksFor(maxL[l], 256));
-      DCG_LAUNCH(DCG_K_SOLVE, "k_sv_lists", (k_sv_lists<BW><<<std::min(n, 1024u), 256, 0, stream>>>(g, breachBuf, svList, svFaces, svCount)));
+      DCG_LAUNCH(DCG_K_SOLVE, "k_sv_lists", (k_sv_lists<BW><<<std::min(n, 1024u), 256, 0, stream>>>(g, breachBuf, svList, svFaces, svCount, cyc)));
       DCG_LAUNCH(DCG_K_SOLVE, "k_sv_mirror_counts",
                  (k_sv_mirror_counts<<<1, 1, 0, stream>>>(svCount, svCountMirrorDev, 2 * L * L)));
     }
@@ -1005,9 +1135,14 @@ struct DCGridSim : SimBase {
     rep.levels = L;
     rep.converged = 1;
     // the guess of a solve in one precision is the pressure field, whatever precision wrote it
-    if (P.solve_precision == DCG_SOLVE_FP32)
+    if (P.solve_precision == DCG_SOLVE_FP32) {
+      DCG_TRY(dctSetup<float>());
       DCG_TRY((solveWithGuess<float, float>()));
-    else if (P.solve_precision == DCG_SOLVE_FP64)
+      warmValid = true;
+      return applyPressure();
+    }
+    DCG_TRY(dctSetup<double>());
+    if (P.solve_precision == DCG_SOLVE_FP64)
       DCG_TRY((solveWithGuess<double, double>()));
     else
       DCG_TRY((solveWithGuess<double, float>()));

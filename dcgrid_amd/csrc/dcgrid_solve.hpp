@@ -9,7 +9,8 @@
 // V-cycle in FP32 whose grids are the level itself, the coarser levels restricted to the
 // ancestors of the level's cells ("reach"), and below the top level a uniform pyramid of the
 // top level (dense by construction). Restriction is the mean of the 8 cells of a restriction
-// group, prolongation the trilinear 27/9/3/1 stencil. Residuals on coarse grids are kept in
+// group, prolongation the trilinear 27/9/3/1 stencil. (A level that covers the domain takes its
+// correction from a direct solve instead, dcgrid_direct.hpp.) Residuals on coarse grids are kept in
 // density units (R / h^2), so restriction is a plain mean and each grid uses its own cell size
 // in the operator.
 //
@@ -160,7 +161,7 @@ __global__ void __launch_bounds__(Geo<BW>::WG) k_sv_reach(DGBase g, int level, u
 }
 
 // Active blocks of the V-cycle grids of every level solve: for lmin <= k, the blocks of level k
-// with breach <= lmin, per colour c, at list[(lmin * 2 + c) * B + offs[k] + i] for
+// with breach <= lmin, for the solves lmin < cyc that run V-cycles, per colour c, at list[(lmin * 2 + c) * B + offs[k] + i] for
 // i < count[(lmin * L + k) * 2 + c] (2 L B entries in all), and beside each entry the block's six
 // face descriptors (faces[entry * 6 + face]), so that a kernel walking a list reads a block's
 // index and its faces together. The order inside a list follows the atomic increments and does
@@ -168,7 +169,7 @@ __global__ void __launch_bounds__(Geo<BW>::WG) k_sv_reach(DGBase g, int level, u
 template <int BW>
 __global__ void __launch_bounds__(256) k_sv_lists(DGBase g, const uint8_t* __restrict__ breach,
                                                   uint32_t* __restrict__ list, int4* __restrict__ faces,
-                                                  uint32_t* __restrict__ count) {
+                                                  uint32_t* __restrict__ count, int cyc) {
   for (int k = 0; k < g.L; k++) {
     const uint32_t n = g.ctl[CTL_LOADS + k];
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
@@ -177,7 +178,7 @@ __global__ void __launch_bounds__(256) k_sv_lists(DGBase g, const uint8_t* __res
       int4 fd[6];
 #pragma unroll
       for (int f = 0; f < 6; f++) fd[f] = g.nd[b * 27 + faceDir(f)];
-      for (int lmin = breach[b]; lmin <= k; lmin++) {
+      for (int lmin = breach[b]; lmin <= k && lmin < cyc; lmin++) {
         const uint32_t slot = atomicAdd(&count[(lmin * g.L + k) * 2 + c], 1u);
         const size_t entry = (size_t)(lmin * 2 + c) * g.B + g.offs[k] + slot;
         list[entry] = b;

@@ -68,7 +68,8 @@ enum { DCG_PROJECT_MULTILEVEL = 0, DCG_PROJECT_LOCAL = 1, DCG_PROJECT_SOLVE = 2 
 
 /* Arithmetic of DCG_PROJECT_SOLVE: FP64 residual / norms / correction update around FP32
  * multigrid cycles with red-black Gauss-Seidel smoothing (MIXED), or everything in FP32 or
- * in FP64. */
+ * in FP64. On FP32 fields, levels that cover the domain (axes up to 1024 cells) are solved directly
+ * by cosine transforms, in FP64 except with FP32; dcg_solve_info.cycles then counts direct solves. */
 enum { DCG_SOLVE_MIXED = 0, DCG_SOLVE_FP32 = 1, DCG_SOLVE_FP64 = 2 };
 
 /* Topology score used by dcg_adapt_topology. */

@@ -188,6 +188,64 @@ def test_precision_variants():
     assert max(res[SOLVE_FP32][0]["rel_residual"]) > 1e-8 or e_32 <= 1e-5
 
 
+# Dense grids around the direct solve's tiles: axes below and past multiples of 32 (padded transform
+# halves), of one block, with partial column tiles (z frequencies, block columns), BW 4 and 8, the
+# longest axis of the 64-line tiles (256), past it (320), of the 32-line tiles (512) and of all (1024).
+DIRECT_CASES = [((64, 96, 160), 8, 3), ((48, 16, 80), 8, 2), ((8, 8, 8), 8, 1), ((24, 8, 40), 8, 1), ((24, 40, 56), 4, 2),
+                ((16, 16, 16), 4, 3), ((20, 4, 12), 4, 1), ((256, 16, 32), 8, 2), ((16, 320, 32), 8, 2),
+                ((16, 32, 512), 8, 2), ((512, 16, 16), 8, 2), ((1024, 16, 16), 8, 2)]
+
+
+@pytest.mark.parametrize("size,bw,levels", DIRECT_CASES)
+def test_dense_levels_against_cosine_transform(size, bw, levels):
+    """Every level of a fully dense grid is a box with Neumann walls: its pressure is the zero-mean
+    solution of scipy's DCT-II in 64 bits, to the rounding of the stored FP32 pressure (1e-7 covers
+    its 6e-8); throughout FP32 to that rounding times the longest axis' condition (n / pi)^2."""
+    from scipy.fft import dctn, idctn
+    p = scenes.reference_params(*size)
+    p.dt, p.dx, p.rdx = 0.1, 1.0, 1.0
+    p.emission_radius = 0.0
+    p.block_width, p.max_levels = bw, levels
+    budget = sum((size[0] // (bw << l)) * (size[1] // (bw << l)) * (size[2] // (bw << l)) for l in range(levels))
+    p.solve_tol = 1e-8
+    g = dcgrid_amd.Simulation("dcgrid", size, p, budget)
+    assert g.info().levels == levels
+    rng = np.random.default_rng(sum(size) + bw)
+    vel = rng.standard_normal((g.field_size("density"), 3)).astype(np.float32)
+    t = g.export_tables()
+    lev, pos = t["block_levels"], t["block_positions"]
+    bits = bw.bit_length() - 1
+    loc = np.arange(bw ** 3)
+    lx, ly, lz = (sum(((loc >> (3 * b + k)) & 1) << b for b in range(bits)) for k in (2, 1, 0))
+    for prec in (SOLVE_MIXED, SOLVE_FP64, SOLVE_FP32):
+        p.solve_precision = prec
+        g.set_params(p)
+        g.import_field("velocity", vel)
+        g.project_solve()
+        rep = g.solve_report()
+        say(size, bw, "precision", prec, "cycles", rep["cycles"], "rel", rep["rel_residual"])
+        if prec != SOLVE_FP32:
+            assert rep["converged"]
+        pre, div = g.export_field("pressure"), g.export_field("divergence")
+        for l in range(levels):
+            n = [v >> l for v in size]
+            b = np.nonzero(lev == l)[0]
+            x, y, z = (pos[b, a][:, None] + o[None, :] for a, o in enumerate((lx, ly, lz)))
+            cells = b[:, None] * bw ** 3 + loc[None, :]
+            box_p, box_d = np.empty(n), np.empty(n)
+            box_p[x, y, z], box_d[x, y, z] = pre[cells], div[cells]
+            lam = sum((4 * np.sin(np.pi * np.arange(n[a]) / (2 * n[a])) ** 2).reshape([-1 if a == k else 1 for k in range(3)])
+                      for a in range(3))
+            lam[0, 0, 0] = 1.0
+            f = dctn(-box_d * float(1 << l) ** 2, type=2, norm="ortho") / lam
+            f[0, 0, 0] = 0.0
+            want = idctn(f, type=2, norm="ortho")
+            err = rel_l2(box_p, want)
+            say("  level", l, n, "pressure rel l2", err)
+            assert err <= (1e-7 if prec != SOLVE_FP32 else 6e-8 * max(1.0, max(n) / np.pi) ** 2 + 1e-6)
+    g.close()
+
+
 def test_step_with_solve_mode():
     """dcg_step with project_mode = DCG_PROJECT_SOLVE: every step's solve converges."""
     kind, size, p, b = workload("cfg2_128")
