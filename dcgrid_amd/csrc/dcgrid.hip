@@ -162,7 +162,10 @@ struct DCGridSim : SimBase {
   unsigned long long* cand1 = nullptr;  // selected destination subblocks of a level
   uint32_t* mcBuf = nullptr;  // sorted move candidates, per-level region at offs[l]
   uint32_t* dcBuf = nullptr;  // sorted destination subblocks, region at offs[l] + l
+  uint32_t *mcKey = nullptr, *dcKey = nullptr;  // their selection keys, same regions
   uint32_t* refList = nullptr;
+  // Keys that fit the selection's LDS (33 words per 32, beside its histogram).
+  static constexpr uint32_t kSelectLdsKeys = 36 * 1024;
   float* stats = nullptr;
   unsigned long long* cellStepCounter = nullptr;
   bool customFluidity = false;
@@ -243,6 +246,8 @@ struct DCGridSim : SimBase {
     DCG_TRY(alloc(&cand1, (size_t)8 * B + 16));
     DCG_TRY(alloc(&mcBuf, (size_t)B + 16));
     DCG_TRY(alloc(&dcBuf, (size_t)B + 16));
+    DCG_TRY(alloc(&mcKey, (size_t)B + 16));
+    DCG_TRY(alloc(&dcKey, (size_t)B + 16));
     DCG_TRY(alloc(&refList, (size_t)8 * B));
     DCG_TRY(alloc(&stats, B));
     DCG_TRY(alloc(&cellStepCounter, 1));
@@ -251,6 +256,8 @@ struct DCGridSim : SimBase {
     std::memcpy(&negBits, &negMax, 4);
     DCG_TRY(fill32(sbs, negBits, (size_t)8 * B + 1));
     DCG_TRY(queryResidentGrids());
+    DCG_HIP(hipFuncSetAttribute((const void*)k_select_pair, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)(kSelectLdsKeys / 32 * 33 + 1) * 4));
     return reset();
   }
   // The grids of the occupancy-sized walks are asked of the runtime here, outside any stream
@@ -356,11 +363,16 @@ struct DCGridSim : SimBase {
     for (int l = 0; l < L - 1; l++) {
       uint32_t* mc = mcBuf + offs[l];
       uint32_t* dc = dcBuf + offs[l] + l;
-      const unsigned rk = blocksFor((size_t)maxL[l] + 1, 256);
-      DCG_LAUNCH(DCG_K_TOPOLOGY, "k_select_pair", (k_select_pair<<<2, 1024, 0, stream>>>(g, l, bs, sbs, cand, cand1)));
-      DCG_LAUNCH(DCG_K_TOPOLOGY, "k_rank_pair", (k_rank_pair<<<dim3(rk, 2), 256, 0, stream>>>(g, l, cand, cand1, mc, dc)));
-      DCG_LAUNCH(DCG_K_TOPOLOGY, "k_match",
-                 (k_match<<<1, 1024, 0, stream>>>(g, l, l == L - 2 ? 1 : 0, mc, dc, bs, sbs)));
+      const unsigned rk = std::min(blocksFor((size_t)maxL[l] + 1, RANK_MINE), 1024u);
+      uint32_t* mk = mcKey + offs[l];
+      uint32_t* dk = dcKey + offs[l] + l;
+      // LDS for the keys of the candidates that the level can have, beyond what registers hold
+      const uint32_t most = 8u * maxL[l + 1], keys = most > 8 * 1024 ? std::min(most, kSelectLdsKeys) : 0u;
+      DCG_LAUNCH(DCG_K_TOPOLOGY, "k_select_pair",
+                 (k_select_pair<<<2, 1024, (size_t)(keys + keys / 32 + 1) * 4, stream>>>(g, l, bs, sbs, cand, cand1, keys)));
+      DCG_LAUNCH(DCG_K_TOPOLOGY, "k_rank_pair",
+                 (k_rank_pair<<<dim3(rk, 2), 256, 0, stream>>>(g, l, cand, cand1, mc, dc, mk, dk)));
+      DCG_LAUNCH(DCG_K_TOPOLOGY, "k_match", (k_match<<<1, 1024, 0, stream>>>(g, l, l == L - 2 ? 1 : 0, dc, mk, dk, bs)));
     }
     // moves coarse to fine; the first launch also clears the hash for the refill (:326-332)
     for (int l = L - 2; l >= 0; l--)

@@ -286,19 +286,22 @@ __device__ __forceinline__ uint32_t selectCount(const DGBase& g, int level, uint
 struct SelectShared {
   uint32_t hist[2048];
   uint32_t sh[17];
-  uint32_t sPrefix, sRem, sCount;
+  uint32_t sPrefix, sRem;
 };
-// Adds 1 to hist[bin] for every active lane of the wavefront. Lanes holding the common key
-// (that of -FLT_MAX scores, shared by every refined or free candidate, often most of them) add
-// with one LDS atomic per wavefront instead of serialising on one bin; the others one atomic
-// each. Called by all lanes of the wavefront.
-__device__ __forceinline__ void histAdd(uint32_t* hist, uint32_t bin, bool active, bool common) {
-  const unsigned long long m = __ballot(active && common);
-  if (active && common) {
-    if ((int)(threadIdx.x & 63) == __ffsll((long long)m) - 1) atomicAdd(&hist[bin], (uint32_t)__popcll(m));
-  } else if (active) {
-    atomicAdd(&hist[bin], 1u);
-  }
+// Adds 1 to hist[bin] for every active lane of the wavefront. The lanes that share the first one's bin
+// (often that of -FLT_MAX scores, most of the candidates) add with one LDS atomic instead of one after
+// the other, the others one each: equal bins among them serialise, but finding them takes longer
+// (three bins collected this way: 53 us for 32768 keys, one 43 us). Called by all lanes of the
+// wavefront.
+__device__ __forceinline__ void histAdd(uint32_t* hist, uint32_t bin, bool active) {
+  const unsigned long long left = __ballot(active);
+  if (left == 0) return;
+  const int lead = __ffsll((long long)left) - 1;
+  const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)bin, lead);
+  const bool shared = active && bin == b;
+  const unsigned long long m = __ballot(shared);
+  if ((int)(threadIdx.x & 63) == lead) atomicAdd(&hist[b], (uint32_t)__popcll(m));
+  if (active && !shared) atomicAdd(&hist[bin], 1u);
 }
 
 // The radix select of selectBody with the thread's keys (a segment of at most KEYS candidates)
@@ -318,8 +321,8 @@ __device__ __forceinline__ void selectInRegisters(uint32_t lo, uint32_t hi, uint
     for (uint32_t j = threadIdx.x; j < 2048; j += T) S.hist[j] = 0;
     __syncthreads();
 #pragma unroll
-    for (uint32_t j = 0; j < KEYS; j++)  // short segments: few equal keys per wavefront, plain atomics
-      if (lo + j < hi && (kr[j] & mask) == prefix) atomicAdd(&S.hist[(kr[j] >> shift) & (nb - 1)], 1u);
+    for (uint32_t j = 0; j < KEYS; j++)
+      histAdd(S.hist, (kr[j] >> shift) & (nb - 1), lo + j < hi && (kr[j] & mask) == prefix);
     __syncthreads();
     const uint32_t a0 = 2 * threadIdx.x < nb ? S.hist[2 * threadIdx.x] : 0;
     const uint32_t a1 = 2 * threadIdx.x + 1 < nb ? S.hist[2 * threadIdx.x + 1] : 0;
@@ -337,10 +340,15 @@ __device__ __forceinline__ void selectInRegisters(uint32_t lo, uint32_t hi, uint
     rem = S.sRem;
     __syncthreads();
   }
-  uint32_t ties = 0;
+  // the winners of a thread together: one scan gives every thread its place
+  uint32_t ties = 0, less = 0;
 #pragma unroll
-  for (uint32_t j = 0; j < KEYS; j++) ties += lo + j < hi && kr[j] == prefix;
+  for (uint32_t j = 0; j < KEYS; j++) {
+    ties += lo + j < hi && kr[j] == prefix;
+    less += lo + j < hi && kr[j] < prefix;
+  }
   const uint32_t tieBase = wgExclusiveScan(ties, S.sh, nullptr);
+  uint32_t slot = wgExclusiveScan(less + min(ties, rem > tieBase ? rem - tieBase : 0u), S.sh, nullptr);
   uint32_t seen = 0;
 #pragma unroll
   for (uint32_t j = 0; j < KEYS; j++) {
@@ -351,16 +359,14 @@ __device__ __forceinline__ void selectInRegisters(uint32_t lo, uint32_t hi, uint
       take = tieBase + seen < rem;
       seen++;
     }
-    if (take) {
-      const uint32_t slot = atomicAdd(&S.sCount, 1u);
-      cand[slot] = ((unsigned long long)kk << 32) | (lo + j);
-    }
+    if (take) cand[slot++] = ((unsigned long long)kk << 32) | (lo + j);
   }
 }
 
 template <int MODE>
-__device__ void selectBody(const DGBase& g, int level, const float* __restrict__ scores,
-                           unsigned long long* __restrict__ cand, SelectShared& S) {
+__device__ __forceinline__ void selectBody(const DGBase& g, int level, const float* __restrict__ scores,
+                           unsigned long long* __restrict__ cand, SelectShared& S, uint32_t* keys,
+                           uint32_t ldsKeys) {
   uint32_t* hist = S.hist;
   uint32_t* sh = S.sh;
   const uint32_t d0 = g.maxL[level], d1 = 8 * g.maxL[level + 1];
@@ -368,8 +374,6 @@ __device__ void selectBody(const DGBase& g, int level, const float* __restrict__
   const uint32_t base = MODE == 0 ? g.offs[level] : 8 * g.offs[level + 1];
   const uint32_t lim = moveLim(g, level);  // the same value in both workgroups of a pair
   if (MODE == 0 && threadIdx.x == 0) g.ctl[CTL_LIM + level] = lim;
-  if (threadIdx.x == 0) S.sCount = 0;
-  __syncthreads();
   const uint32_t k = selectCount<MODE>(g, level, lim);
   if (k == 0) return;
   const uint32_t T = blockDim.x;
@@ -394,7 +398,26 @@ __device__ void selectBody(const DGBase& g, int level, const float* __restrict__
     selectInRegisters<SELECT_REG_KEYS>(lo, hi, k, key32, cand, S);
     return;
   }
-  const uint32_t common = MODE == 0 ? blockKey(-FLT_MAX) : subKey(-FLT_MAX);
+  // Longer segments: the keys are read once, coalesced, into LDS where they fit (ldsKeys, the launch's
+  // capacity), else read again in every pass. Entry i of the LDS array sits at i + i / 32, so that
+  // consecutive candidates and a thread's segment are both spread over the banks. Measured (MI355X,
+  // 32768 subblocks of 4^3 blocks): about 80 us with every pass reading its segments from memory, 43 us.
+  const bool inLds = nA <= ldsKeys;
+  if (inLds) {
+    constexpr uint32_t U = 16;  // loads in flight per thread
+    for (uint32_t i0 = threadIdx.x; i0 < nA; i0 += U * T) {
+      uint32_t v[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) v[u] = key32(min(i0 + u * T, nA - 1));
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) {
+        const uint32_t i = i0 + u * T;
+        if (i < nA) keys[i + (i >> 5)] = v[u];
+      }
+    }
+    __syncthreads();
+  }
+  auto keyOf = [&](uint32_t i) -> uint32_t { return inLds ? keys[i + (i >> 5)] : key32(i); };
   // Radix select on key32: 11 + 11 + 10 bits.
   uint32_t prefix = 0, mask = 0, rem = k;
   for (int pass = 0; pass < 3; pass++) {
@@ -402,11 +425,11 @@ __device__ void selectBody(const DGBase& g, int level, const float* __restrict__
     const uint32_t nb = pass == 2 ? 1024u : 2048u;
     for (uint32_t j = threadIdx.x; j < 2048; j += T) hist[j] = 0;
     __syncthreads();
-#pragma unroll 1
-    for (uint32_t j = 0; j < seg; j++) {  // the same trip count in every lane
-      const uint32_t i = lo + j;
-      const uint32_t kk = i < hi ? key32(i) : 0u;
-      histAdd(hist, (kk >> shift) & (nb - 1), i < hi && (kk & mask) == prefix, kk == common);
+#pragma unroll 4
+    for (uint32_t j = 0; j < seg; j++) {  // the same trip count in every lane; any order will do
+      const uint32_t i = j * T + threadIdx.x;
+      const uint32_t kk = i < nA ? keyOf(i) : 0u;
+      histAdd(hist, (kk >> shift) & (nb - 1), i < nA && (kk & mask) == prefix);
     }
     __syncthreads();
     const uint32_t a0 = 2 * threadIdx.x < nb ? hist[2 * threadIdx.x] : 0;
@@ -425,60 +448,83 @@ __device__ void selectBody(const DGBase& g, int level, const float* __restrict__
     rem = S.sRem;
     __syncthreads();
   }
-  // prefix = key32 of the k-th smallest; take all smaller keys and the first `rem` ties.
-  uint32_t ties = 0;
-  for (uint32_t i = lo; i < hi; i++) ties += key32(i) == prefix;
+  // prefix = key32 of the k-th smallest; take all smaller keys and the first `rem` ties, the
+  // winners of a thread's segment together (one scan gives every thread its place)
+  uint32_t ties = 0, less = 0;
+#pragma unroll 4
+  for (uint32_t i = lo; i < hi; i++) {
+    const uint32_t kk = keyOf(i);
+    ties += kk == prefix;
+    less += kk < prefix;
+  }
   const uint32_t tieBase = wgExclusiveScan(ties, sh, nullptr);
+  const uint32_t mine = less + min(ties, rem > tieBase ? rem - tieBase : 0u);
+  uint32_t slot = wgExclusiveScan(mine, sh, nullptr);
   uint32_t seen = 0;
   for (uint32_t i = lo; i < hi; i++) {
-    const uint32_t kk = key32(i);
+    const uint32_t kk = keyOf(i);
     bool take = kk < prefix;
     if (kk == prefix) {
       take = tieBase + seen < rem;
       seen++;
     }
-    if (take) {
-      const uint32_t slot = atomicAdd(&S.sCount, 1u);
-      cand[slot] = ((unsigned long long)kk << 32) | i;
-    }
+    if (take) cand[slot++] = ((unsigned long long)kk << 32) | i;
   }
 }
 // Both selections of one level in one launch: workgroup 0 the move candidates (block scores),
 // workgroup 1 the destination subblocks (subblock scores); they read only scores and loads.
+// ldsKeys: candidates whose keys fit the launch's dynamic LDS (33 words per 32).
 __global__ void __launch_bounds__(1024) k_select_pair(DGBase g, int level, const float* __restrict__ bs,
                                                       const float* __restrict__ sbs, unsigned long long* __restrict__ cand0,
-                                                      unsigned long long* __restrict__ cand1) {
+                                                      unsigned long long* __restrict__ cand1, uint32_t ldsKeys) {
   __shared__ SelectShared S;
+  extern __shared__ uint32_t selectKeys[];
   if (blockIdx.x == 0)
-    selectBody<0>(g, level, bs, cand0, S);
+    selectBody<0>(g, level, bs, cand0, S, selectKeys, ldsKeys);
   else
-    selectBody<1>(g, level, sbs, cand1, S);
+    selectBody<1>(g, level, sbs, cand1, S, selectKeys, ldsKeys);
 }
 
-// Exact position of every selected candidate (keys are unique): out[rank] = base + position.
-// blockIdx.y selects the list: 0 move candidates -> mc, 1 destination subblocks -> dc.
+// Exact position of every selected candidate (keys are unique): out[rank] = base + position, with its
+// key32 beside it for the match. blockIdx.y selects the list: 0 move candidates -> mc, 1 destination
+// subblocks -> dc. A wavefront ranks RANK_PER candidates, its lanes each against a 64th of all: the
+// comparisons (k^2) spread over the whole chip instead of the k / 256 workgroups of one thread per
+// candidate, and every value loaded is compared RANK_PER times. Measured (MI355X, 7320
+// candidates): about 100 -> 18 us.
+constexpr uint32_t RANK_PER = 4, RANK_MINE = 256 / 64 * RANK_PER;
 __global__ void __launch_bounds__(256) k_rank_pair(DGBase g, int level, const unsigned long long* __restrict__ cand0,
                                                    const unsigned long long* __restrict__ cand1,
-                                                   uint32_t* __restrict__ mc, uint32_t* __restrict__ dc) {
-  __shared__ unsigned long long tile[1024];
+                                                   uint32_t* __restrict__ mc, uint32_t* __restrict__ dc,
+                                                   uint32_t* __restrict__ mcKey, uint32_t* __restrict__ dcKey) {
   const int mode = blockIdx.y;
   const uint32_t lim = g.ctl[CTL_LIM + level];
   const uint32_t k = mode == 0 ? selectCount<0>(g, level, lim) : selectCount<1>(g, level, lim);
-  const unsigned long long* cand = mode == 0 ? cand0 : cand1;
-  uint32_t* out = mode == 0 ? mc : dc;
+  const unsigned long long* __restrict__ cand = mode == 0 ? cand0 : cand1;
   const uint32_t base = mode == 0 ? g.offs[level] : 8 * g.offs[level + 1];
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (blockIdx.x * 256 >= k) return;
-  const unsigned long long mine = i < k ? cand[i] : ~0ull;
-  uint32_t rank = 0;
-  for (uint32_t t0 = 0; t0 < k; t0 += 1024) {
-    for (uint32_t j = threadIdx.x; j < 1024; j += 256) tile[j] = t0 + j < k ? cand[t0 + j] : ~0ull;
-    __syncthreads();
-    const uint32_t m = min(1024u, k - t0);
-    for (uint32_t j = 0; j < m; j++) rank += tile[j] < mine;
-    __syncthreads();
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (uint32_t i0 = blockIdx.x * RANK_MINE + wave * RANK_PER; i0 < k; i0 += gridDim.x * RANK_MINE) {
+    unsigned long long mine[RANK_PER];
+    uint32_t rank[RANK_PER];
+#pragma unroll
+    for (uint32_t c = 0; c < RANK_PER; c++) {
+      mine[c] = cand[min(i0 + c, k - 1)];
+      rank[c] = 0;
+    }
+#pragma unroll 8
+    for (uint32_t j = lane; j < k; j += 64) {
+      const unsigned long long other = cand[j];
+#pragma unroll
+      for (uint32_t c = 0; c < RANK_PER; c++) rank[c] += other < mine[c];
+    }
+#pragma unroll
+    for (uint32_t c = 0; c < RANK_PER; c++) {
+      for (int o = 32; o > 0; o >>= 1) rank[c] += __shfl_xor(rank[c], o, 64);
+      if (lane == c && i0 + c < k) {
+        (mode == 0 ? mc : dc)[rank[c]] = base + (uint32_t)(mine[c] & 0xFFFFFFFFu);
+        (mode == 0 ? mcKey : dcKey)[rank[c]] = (uint32_t)(mine[c] >> 32);
+      }
+    }
   }
-  if (i < k) out[rank] = base + (uint32_t)(mine & 0xFFFFFFFFu);
 }
 
 // Match loop of moveBlocks (fluid_simulation_dcgrid.cu:410-421). The conditions are monotone
@@ -491,9 +537,12 @@ __device__ __forceinline__ void totalMoves(const DGBase& g, int level, uint32_t 
   for (int l = 0; l < level; l++) s += g.ctl[CTL_MOVES + l];
   g.ctl[CTL_TOTAL_MOVES] = s;
 }
-__global__ void __launch_bounds__(1024) k_match(DGBase g, int level, int last, const uint32_t* __restrict__ mc,
-                                                const uint32_t* __restrict__ dc, float* __restrict__ bs,
-                                                const float* __restrict__ sbs) {
+// The scores are those of the keys (blockKey, subKey inverted; a negative block score's key reads as
+// NaN and fails the test as the score does, and the sign of a zero subblock score does not matter
+// to it).
+__global__ void __launch_bounds__(1024) k_match(DGBase g, int level, int last, const uint32_t* __restrict__ dc,
+                                                const uint32_t* __restrict__ mcKey, const uint32_t* __restrict__ dcKey,
+                                                float* __restrict__ bs) {
   __shared__ uint32_t sFail;
   const uint32_t lim = g.ctl[CTL_LIM + level];
   if (lim == 0) {
@@ -505,10 +554,17 @@ __global__ void __launch_bounds__(1024) k_match(DGBase g, int level, int last, c
   }
   if (threadIdx.x == 0) sFail = lim;
   __syncthreads();
+  uint32_t fail = lim;  // the thread's first failing position
   for (uint32_t m = threadIdx.x; m < lim; m += blockDim.x) {
-    const float a = bs[mc[m]], b = sbs[dc[m]];
-    if (!(a >= 0.f && b >= 0.f && a < b)) atomicMin(&sFail, m);
+    const uint32_t u = ~dcKey[m];
+    const float a = __uint_as_float(mcKey[m]), b = __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
+    if (!(a >= 0.f && b >= 0.f && a < b)) {
+      fail = m;
+      break;
+    }
   }
+  for (int o = 32; o > 0; o >>= 1) fail = min(fail, (uint32_t)__shfl_xor((int)fail, o, 64));
+  if ((threadIdx.x & 63) == 0 && fail < lim) atomicMin(&sFail, fail);
   __syncthreads();
   const uint32_t M = sFail;
   const uint32_t d1 = 8 * g.maxL[level + 1];

@@ -152,6 +152,26 @@ def test_dcgrid_steps_bitwise_vs_fp32_oracle(name):
         assert g.debug_stats() == c.debug_stats()
 
 
+# Move selections by the candidates of a level: keys in registers (up to 8192; 4096 subblocks of the
+# dense level 1: 512), in LDS (32768 with many and few moves) and beyond it (64000, 46656).
+@pytest.mark.parametrize("n,levels,budget", [(64, 3, 900), (128, 3, 4096 + 512 + 4500), (128, 3, 4096 + 512 + 1200),
+                                             (160, 3, 8000 + 1000 + 9000), (144, 3, 5832 + 729 + 6000)])
+def test_dcgrid_selection_paths(n, levels, budget):
+    """Topology after reset and two steps (moves on the sparse level 0, geometric scores with many
+    equal leading digits) equals the oracle's, block by block."""
+    p = scenes.reference_params(n)
+    p.max_levels = levels
+    g = dcgrid_amd.Simulation("dcgrid", (n, n, n), p, budget)
+    c = oracle.OracleSim("dcgrid", (n, n, n), p, budget, precision=32)
+    assert_tables_equal(g, c)
+    for _ in range(2):
+        g.step(1)
+        c.step(1)
+        assert_tables_equal(g, c)
+    g.close()
+    c.close()
+
+
 @pytest.mark.parametrize("name", ["cfg1_64", "ref64_bw4_solids"])
 def test_dcgrid_project_local_bitwise(name):
     """projectLocal (fluid_simulation_dcgrid.cu:296-311): divergence, project_local_pairs Jacobi
