@@ -344,6 +344,33 @@ def test_uniform_fused_sweeps_bitwise(size, mode, pairs):
     c.close()
 
 
+# Samples whose corners all lie in the domain and samples across every face, edge and corner of it, on
+# extents of 1 and 2 (no inner sample), a row of one wavefront and one past it; cells and displacements
+# of several cells in every direction, and (large) back traces from far outside.
+@pytest.mark.parametrize("size", [(1, 1, 1), (1, 5, 7), (2, 2, 2), (3, 1, 4), (64, 3, 2), (65, 9, 8)])
+@pytest.mark.parametrize("speed", [0.3, 4.0, 1e4])
+def test_uniform_advection_samples_bitwise(size, speed):
+    """Both advections equal the oracle's bit for bit whichever corners a sample has."""
+    p = scenes.reference_params(*size, kind="uniform")
+    p.dt, p.dx, p.rdx = 1.0, 1.0, 1.0
+    g = dcgrid_amd.Simulation("uniform", size, p)
+    c = oracle.OracleSim("uniform", size, p, precision=32)
+    n = size[0] * size[1] * size[2]
+    rng = np.random.default_rng(n)
+    vel = (rng.standard_normal((n, 3)) * speed).astype(np.float32)
+    den = rng.random(n).astype(np.float32)
+    for s in (g, c):
+        s.import_field("velocity", vel)
+        s.import_field("density", den)
+        s.import_field("temperature", den[::-1].copy())
+        s.advect_velocity()
+        s.advect_density()
+    for f in ("velocity", "density", "temperature"):
+        assert bitwise(g.export_field(f), c.export_field(f)), (size, speed, f)
+    g.close()
+    c.close()
+
+
 def test_uniform_fp64_per_step():
     size, p, _ = uniform_workload("cfg0_32")
     g = dcgrid_amd.Simulation("uniform", size, p)
