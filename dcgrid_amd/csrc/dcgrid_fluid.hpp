@@ -74,12 +74,12 @@ template <int BW>
 __device__ __forceinline__ uint32_t slotStride() {
   return gridDim.x * Geo<BW>::BPW;
 }
-template <int BW>
+// N: threads per block.
+template <int BW, int N = Geo<BW>::BV>
 __device__ __forceinline__ BlockCtx<BW> slotCtx(const DGBase& g, int level, uint32_t base, uint32_t total) {
-  constexpr int BV = Geo<BW>::BV;
   BlockCtx<BW> c;
-  c.sub = threadIdx.x / BV;
-  c.t = threadIdx.x % BV;
+  c.sub = threadIdx.x / N;
+  c.t = threadIdx.x % N;
   const uint32_t slot = base + c.sub;
   c.valid = slot < total;
   c.level = 0;
@@ -671,7 +671,7 @@ struct TileSample {
     const int t = (((qx >> (BB - 1)) & 1) << 2) | (((qy >> (BB - 1)) & 1) << 1) | ((qz >> (BB - 1)) & 1);
     if (chi8[t] != NFU) return false;
     scale = 1 << lb;
-    const float scaleInv = 1.f / (float)scale;
+    const float scaleInv = __uint_as_float((uint32_t)(127 - lb) << 23);  // 1 / scale
     const float x = px * scaleInv - .5f, y = py * scaleInv - .5f, z = pz * scaleInv - .5f;
     const float xf = floorf(x), yf = floorf(y), zf = floorf(z);
     const float dx = x - xf, dy = y - yf, dz = z - zf;
@@ -714,20 +714,73 @@ struct TileSample {
   }
 };
 
+// op(tile entry, cell) for the border entries of block b's apron that thread t of the block's N stages:
+// faces, edges and corners. A thread's entries are resolved together: the neighbours' descriptor words
+// first, all at once, then the fields' loads; an entry toward a same-level block needs no more than the
+// word, entries toward a coarser block or outside the domain take borderApronCell. Walking all 1000
+// entries of the grown block in rounds, each a descriptor and then the fields, cost a chain of eight
+// memory latencies per block and 70 instructions per entry (see k_advect_density for the times).
+template <int BW, int N, class Op>
+__device__ __forceinline__ void forBorder(const DGBase& g, uint32_t b, int t, Op op) {
+  constexpr int A = Geo<BW>::A, BB = Geo<BW>::BB, BV = Geo<BW>::BV, FACE = Geo<BW>::FACE, EDGE = 12 * BW;
+  constexpr int COUNT = FACE + EDGE + 8, PER = (COUNT + N - 1) / N;
+  uint32_t e[PER], src[PER];  // e: tile entry | direction << 10 | same-level local cell << 15; ~0: none
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const int f = t + j * N;
+    int ai, aj, ak;
+    if (f < FACE) {
+      faceCell<BW>(f, ai, aj, ak);
+    } else if (f < FACE + EDGE) {  // four edges along each axis
+      const int h = f - FACE, axis = h / (4 * BW), k = (h / BW) % 4, v = 1 + h % BW;
+      const int lo = (k & 1) ? BW + 1 : 0, hi = (k & 2) ? BW + 1 : 0;
+      ai = axis == 0 ? v : lo;
+      aj = axis == 1 ? v : (axis == 0 ? lo : hi);
+      ak = axis == 2 ? v : hi;
+    } else {
+      const int k = f - FACE - EDGE;
+      ai = (k & 4) ? BW + 1 : 0;
+      aj = (k & 2) ? BW + 1 : 0;
+      ak = (k & 1) ? BW + 1 : 0;
+    }
+    const int dx = ai == 0 ? -1 : (ai == BW + 1 ? 1 : 0);
+    const int dy = aj == 0 ? -1 : (aj == BW + 1 ? 1 : 0);
+    const int dz = ak == 0 ? -1 : (ak == BW + 1 ? 1 : 0);
+    const uint32_t same = loc<BB>((ai - 1) & (BW - 1), (aj - 1) & (BW - 1), (ak - 1) & (BW - 1));
+    const uint32_t dir = (uint32_t)dirIndex(dx, dy, dz);
+    e[j] = f < COUNT ? (uint32_t)((ai * A + aj) * A + ak) | dir << 10 | same << 15 : ~0u;
+    src[j] = f < COUNT ? (uint32_t)g.nd[b * 27 + dir].x : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    if (e[j] == ~0u) continue;
+    const int a = (int)(e[j] & 1023u);
+    src[j] = (src[j] >> 27) == 0 ? src[j] * BV + (e[j] >> 15) : borderApronCell<BW>(g, b, a / (A * A), (a / A) % A, a % A);
+  }
+#pragma unroll
+  for (int j = 0; j < PER; j++)
+    if (e[j] != ~0u) op((int)(e[j] & 1023u), src[j]);
+}
+// Whether every cell of block b's apron lies in the domain: no boundary condition can apply to a
+// sample of its tile (p0: the block's origin in cells of its level).
+template <int BW>
+__device__ __forceinline__ bool apronInside(const dcg_params& P, int3 p0, int level) {
+  return p0.x > 0 && p0.y > 0 && p0.z > 0 && (p0.x + BW) << level < P.gx && (p0.y + BW) << level < P.gy &&
+         (p0.z + BW) << level < P.gz;
+}
+
 // Visits the whole apron of block b ((BW+2)^3 entries, edges and corners included) for thread t
-// of the N = BV / CPT threads that handle the block: op(a, cell) for the thread's CPT interior
-// cells (t + j N) and for its share of the border entries, with the cell of each entry resolved
-// once (apronCell) however many fields are staged from it.
+// of the N threads that handle the block: op(a, cell) for the thread's CPT interior cells (t + j N)
+// and for its border entries, with the cell of each entry resolved once however many fields are
+// staged from it.
 template <int BW, int CPT, class Op>
 __device__ __forceinline__ void forApron(const DGBase& g, uint32_t b, int t, Op op) {
-  constexpr int BV = Geo<BW>::BV, A = Geo<BW>::A, A3 = Geo<BW>::A3, N = BV / CPT;
+  constexpr int BV = Geo<BW>::BV, N = BV / CPT;
 #pragma unroll
   for (int j = 0; j < CPT; j++) op(apronIndexOfLocal<BW>(t + j * N), b * BV + t + j * N);
-  for (int a = t; a < A3; a += N) {
-    const int ai = a / (A * A), aj = (a / A) % A, ak = a % A;
-    if (ai > 0 && ai <= BW && aj > 0 && aj <= BW && ak > 0 && ak <= BW) continue;
-    op(a, borderApronCell<BW>(g, b, ai, aj, ak));
-  }
+  int tr = t;
+  asm volatile("" : "+v"(tr));  // entries resolved anew for every block: kept across blocks they spill registers
+  forBorder<BW, N>(g, b, tr, op);
 }
 
 // Advection workgroup shape. The advection kernels hold ~90-100 VGPRs (5 waves per SIMD), so a
@@ -736,15 +789,20 @@ __device__ __forceinline__ void forApron(const DGBase& g, uint32_t b, int t, Op 
 // BV / CPT threads with CPT cells each, one cell after the other: more blocks resident at the
 // same register count (two cells per thread: four resident blocks per CU; four cells per thread
 // measured slower). BW 4 keeps four blocks of 64 threads.
+// What a block costs besides is the chain of loads before its samples and the instructions around
+// them: resolving the apron's border in one batch (forBorder) and leaving out the boundary conditions
+// for blocks whose apron lies in the domain took, for the terrain of 1024 x 256 x 1024 cells, the
+// density, temperature and vapor from 7260 to 5690 us and the velocity from 5870 to 4540; on the 256^3
+// plume 18.5 to 16.6 and 16.5 to 14.5. (The border's entries kept in registers from block to block:
+// 6655 and 5357, twelve spilled registers.)
 template <int BW>
 struct AdvGeo {
   static constexpr int CPT = BW == 8 ? 2 : 1;
   static constexpr int WG = Geo<BW>::WG / CPT;
 };
 // Minimum waves per SIMD asked of the compiler: 5 for BW 8 (at most 96 VGPRs, five blocks
-// resident per CU). The variants without fluidity-weighted temperature or vapor fit without
-// spilling; the terrain variants (fluidity with buoyancy, moist density) spill a few VGPRs on
-// their cross-block path and still run faster than at four waves.
+// resident per CU). All fit without spilling but the moist density and, with 16-bit storage, the
+// terrain's velocity: one VGPR each, on the cross-block path.
 template <int BW>
 struct AdvWaves {
   static constexpr int value = BW == 8 ? 5 : 1;
@@ -763,7 +821,7 @@ __global__ void __launch_bounds__(AdvGeo<BW>::WG, (AdvWaves<BW>::value)) k_advec
   const uint32_t total = slotTotal(g, -1);
   for (uint32_t base = firstSlot<BW>(); base < total; base += slotStride<BW>()) {
     __syncthreads();  // the previous block's tiles are no longer read
-    const BlockCtx<BW> c = slotCtx<BW>(g, -1, base, total);  // c.t: the thread's first cell
+    const BlockCtx<BW> c = slotCtx<BW, N>(g, -1, base, total);  // c.t: the thread's first cell
     float3* vt = vtiles[c.sub];
     float* ft = FLUIDITY ? ftiles[c.sub] : nullptr;
     uint32_t* chi8 = chis[c.sub];
@@ -779,6 +837,7 @@ __global__ void __launch_bounds__(AdvGeo<BW>::WG, (AdvWaves<BW>::value)) k_advec
     __syncthreads();
     if (!c.valid) continue;
     const int level = c.level;
+    const bool inside = apronInside<BW>(P, p0, level);
 #pragma unroll 1
     for (int j = 0; j < CPT; j++) {
       const int t = c.t + j * N;
@@ -798,7 +857,14 @@ __global__ void __launch_bounds__(AdvGeo<BW>::WG, (AdvWaves<BW>::value)) k_advec
       float3 acc = make_float3(0.f, 0.f, 0.f);
       TileSample<BW, FLUIDITY> ts;
       if (ts.init(g, px, py, pz, chi8, p0, level, ft)) {
-        if (!ts.zero) {
+        if (ts.zero) {
+        } else if (inside) {
+#pragma unroll
+          for (int k = 0; k < 8; k++) {
+            const float3 vk = vt[ts.a0 + ts.off(k)];
+            acc = k == 0 ? f3mul(vk, ts.w[0]) : f3add(acc, f3mul(vk, ts.w[k]));
+          }
+        } else {
 #pragma unroll
           for (int k = 0; k < 8; k++) {
             const float3 vk = velocityBC(P, vt[ts.a0 + ts.off(k)], ts.x0 + ((k >> 2) & 1), ts.y0 + ((k >> 1) & 1),
@@ -845,7 +911,7 @@ __global__ void __launch_bounds__(AdvGeo<BW>::WG, (AdvWaves<BW>::value)) k_advec
   const uint32_t total = slotTotal(g, -1);
   for (uint32_t base = firstSlot<BW>(); base < total; base += slotStride<BW>()) {
     __syncthreads();  // the previous block's tiles are no longer read
-    const BlockCtx<BW> c = slotCtx<BW>(g, -1, base, total);  // c.t: the thread's first cell
+    const BlockCtx<BW> c = slotCtx<BW, N>(g, -1, base, total);  // c.t: the thread's first cell
     float* dt_ = dtiles[c.sub];
     float* tt = SRC ? ttiles[c.sub] : nullptr;
     float* vt = MOIST ? vtiles[c.sub] : nullptr;
@@ -867,6 +933,7 @@ __global__ void __launch_bounds__(AdvGeo<BW>::WG, (AdvWaves<BW>::value)) k_advec
     __syncthreads();
     if (!c.valid) continue;
     const int level = c.level;
+    const bool inside = apronInside<BW>(P, p0, level);
 #pragma unroll 1
     for (int j = 0; j < CPT; j++) {
       const int t = c.t + j * N;
@@ -885,7 +952,16 @@ __global__ void __launch_bounds__(AdvGeo<BW>::WG, (AdvWaves<BW>::value)) k_advec
       float q = 0.f, tq = 0.f, vq = 0.f;
       TileSample<BW, FLUIDITY> ts;
       if (ts.init(g, px, py, pz, chi8, p0, level, ft)) {
-        if (!ts.zero) {
+        if (ts.zero) {
+        } else if (inside) {
+#pragma unroll
+          for (int k = 0; k < 8; k++) {
+            const int e = ts.a0 + ts.off(k);
+            q = k == 0 ? dt_[e] * ts.w[0] : q + dt_[e] * ts.w[k];
+            if (SRC) tq = k == 0 ? tt[e] * ts.w[0] : tq + tt[e] * ts.w[k];
+            if (MOIST) vq = k == 0 ? vt[e] * ts.w[0] : vq + vt[e] * ts.w[k];
+          }
+        } else {
 #pragma unroll
           for (int k = 0; k < 8; k++) {
             const int cx = ts.x0 + ((k >> 2) & 1), cy = ts.y0 + ((k >> 1) & 1), cz = ts.z0 + (k & 1);
