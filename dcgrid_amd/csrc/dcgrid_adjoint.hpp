@@ -734,43 +734,76 @@ __global__ void __launch_bounds__(Geo<BW>::WG) k_da_grad_T(DG g, dcg_params P, i
 // run of sweeps the first launch adds to lin (accumulate = 1: lin holds what finer levels and
 // later stages passed to it), the later ones store (their lin was the previous launch's lout,
 // cleared in the forward sense); coarser cells always accumulate.
+// A launch over a few thousand blocks is a chain of memory latencies, so a thread loads its own cell of
+// all three arrays and the descriptor of its face entry at once and the entry's value next, and passes
+// on what that one entry owes an outside or coarser cell. With the descriptors staged in LDS first, the
+// sums read only where they are stored, and every border cell testing its six directions, the 256^3
+// scene's launch took 9.85 us instead of 7.6.
 template <int BW>
 __global__ void __launch_bounds__(Geo<BW>::WG) k_da_jacobi_T(DGBase g, int level, const float* __restrict__ lout,
                                                              float* __restrict__ lin, float* __restrict__ ld,
                                                              float alpha, int accumulate) {
-  constexpr int BV = Geo<BW>::BV, A3 = Geo<BW>::A3, BPW = Geo<BW>::BPW, BB = Geo<BW>::BB;
+  constexpr int BV = Geo<BW>::BV, A3 = Geo<BW>::A3, BPW = Geo<BW>::BPW, BB = Geo<BW>::BB, FACE = Geo<BW>::FACE;
+  constexpr int FPT = (FACE + BV - 1) / BV;  // face entries per thread
   __shared__ float tiles[BPW][A3];
   __shared__ float accs[BPW][BV];
-  __shared__ int4 nds[BPW][6];
   const uint32_t total = slotTotal(g, level);
   for (uint32_t base = firstSlot<BW>(); base < total; base += slotStride<BW>()) {
     __syncthreads();
     const BlockCtx<BW> c = slotCtx<BW>(g, level, base, total);
     float* tile = tiles[c.sub];
     float* acc = accs[c.sub];
-    acc[c.t] = 0.f;
-    if (c.valid) Faces<BW>::stage(g, nds[c.sub], c.b, c.t);
-    __syncthreads();
-    const Faces<BW> fa{nds[c.sub], c.b};
-    if (c.valid) fa.stageSameLevel(tile, c.t, [&](uint32_t i) { return lout[i] / 6.f; });
-    __syncthreads();
     const int a = apronIndexOfLocal<BW>(c.t);
     const uint32_t cell = c.b * BV + c.t;
+    float G = 0.f, d0 = 0.f, i0 = 0.f;
+    uint32_t sh[FPT], nb[FPT];  // of the thread's face entries: level shift and cell
+    int in[FPT];                // and the tile entry of the block's cell beside them
+    acc[c.t] = 0.f;
     if (c.valid) {
-      const float G = tile[a];
-      if (G != 0.f) {
-        ld[cell] += -alpha * G;
-        int lx, ly, lz;
-        locPos<BB>((uint32_t)c.t, lx, ly, lz);
+      float fv[FPT];
+      int fa[FPT];
+      int4 q[FPT];
+      G = lout[cell];
+      d0 = ld[cell];
+      if (accumulate) i0 = lin[cell];
 #pragma unroll
-        for (int k = 0; k < 6; k++) {
-          uint32_t nb;
-          const int kind = fa.neighbour(lx, ly, lz, k, nb);
-          if (kind == NB_OUT)
-            ldsAdd(&acc[localOf<BW>(nb)], G);
-          else if (kind == NB_COARSER)
-            atomicAddF(&lin[nb], G);
-        }
+      for (int j = 0; j < FPT; j++) {
+        const int fc = c.t + j * BV < FACE ? c.t + j * BV : FACE - 1;
+        q[j] = g.nd[c.b * 27 + Faces<BW>::dirOf(fc / (BW * BW))];
+      }
+#pragma unroll
+      for (int j = 0; j < FPT; j++) {
+        const int fc = c.t + j * BV < FACE ? c.t + j * BV : FACE - 1;
+        int ai, aj, ak;
+        faceCell<BW>(fc, ai, aj, ak);
+        const int ci = clampi(ai, 1, BW), cj = clampi(aj, 1, BW), ck = clampi(ak, 1, BW);
+        fa[j] = tix<BW>(ai, aj, ak);
+        in[j] = tix<BW>(ci, cj, ck);
+        sh[j] = ndShift(q[j]);
+        if (sh[j] == ND_OUT)
+          nb[j] = c.b * BV + (q[j].y ? loc<BB>(ci & (BW - 1), cj & (BW - 1), ck & (BW - 1)) : loc<BB>(ci - 1, cj - 1, ck - 1));
+        else
+          nb[j] = ndBlock(q[j]) * BV + loc<BB>((ai - 1 - q[j].y) >> sh[j], (aj - 1 - q[j].z) >> sh[j], (ak - 1 - q[j].w) >> sh[j]);
+        fv[j] = lout[sh[j] == 0 ? nb[j] : cell];
+      }
+      G = G / 6.f;
+      tile[a] = G;
+#pragma unroll
+      for (int j = 0; j < FPT; j++)
+        if (c.t + j * BV < FACE) tile[fa[j]] = sh[j] == 0 ? fv[j] / 6.f : 0.f;
+    }
+    __syncthreads();
+    if (c.valid) {
+      if (G != 0.f) ld[cell] = d0 + -alpha * G;
+#pragma unroll
+      for (int j = 0; j < FPT; j++) {
+        if (c.t + j * BV >= FACE || sh[j] == 0) continue;
+        const float Gi = tile[in[j]];
+        if (Gi == 0.f) continue;
+        if (sh[j] == ND_OUT)
+          ldsAdd(&acc[localOf<BW>(nb[j])], Gi);
+        else
+          atomicAddF(&lin[nb[j]], Gi);
       }
     }
     __syncthreads();
@@ -778,11 +811,10 @@ __global__ void __launch_bounds__(Geo<BW>::WG) k_da_jacobi_T(DGBase g, int level
       int e[6];
       faceEntries<BW>(a, e);
       const float sum = tile[e[0]] + tile[e[1]] + tile[e[2]] + tile[e[3]] + tile[e[4]] + tile[e[5]] + acc[c.t];
-      lin[cell] = accumulate ? lin[cell] + sum : sum;
+      lin[cell] = accumulate ? i0 + sum : sum;
     }
   }
 }
-
 // k_da_jacobi_T on a dense level (l >= S): every face neighbour is a same-level cell or, outside
 // the domain, the cell itself (dense blocks keep the clamped-own-cell form), so the transposed
 // sweep is the forward stencil applied to lout/6, staged like the forward dense sweep (faces from
