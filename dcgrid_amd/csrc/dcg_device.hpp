@@ -249,11 +249,6 @@ __device__ __forceinline__ float sixthFast(float x) {
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(e, r, q), 6.f, x);
 }
 __device__ __forceinline__ bool sixthUnsure(float q) { return __builtin_amdgcn_classf(q, 0x010 | 0x080); }
-__device__ __forceinline__ float sixth(float x) {
-  float q = sixthFast(x);
-  if (sixthUnsure(q)) q = x / 6.f;
-  return q;
-}
 
 // XCD-aware remap of a linear workgroup id: consecutive ids are dispatched round-robin over the
 // 8 XCDs of MI355X; this maps them so each XCD works on a contiguous range (shared L2 reuse).

@@ -19,7 +19,7 @@
 // 69 that the instruction alone reaches), y back 32, z back 75 us; 64^3 and less 4-9 us, latency. Against
 // the V-cycles of such a level (seven to nine, to 1e-8) it leaves one step at 1e-13: a projection of
 // 256 x 128 x 256 cells on three dense levels 6.24 -> 0.96 ms, of 512 x 128 x 512 on four 19.2 -> 4.1 ms,
-// of configuration 2 (two of four levels dense) 4.82 -> 2.19 ms. In FP32 throughout, four to five
+// of 512^3 cells in 32768 blocks of 8^3 (two of four levels dense) 4.82 -> 2.19 ms. In FP32 throughout, four to five
 // steps stall where the V-cycles' seven to nine did.
 #pragma once
 
