@@ -87,7 +87,7 @@ def step_bytes(info, params, uniform=False):
         act = int(info.active_cells)
         sweeps = 2 * (params.project_local_pairs if params.project_mode == 1 else params.project_level_pairs)
         return act * (pc["advect_velocity"] + pc["advect_density"] + pc["divergence"] + pc["apply_pressure"] +
-                      12 * sweeps)
+                      12 * -(-sweeps // 4))  # a launch of up to four half-sweeps passes over the level once
     bv = int(info.block_width) ** 3
     L = int(info.levels)
     src = params.source_mode != 0
@@ -508,7 +508,7 @@ def main():
                 else:
                     bytes_ = jacobi_bytes(info1, p)[0] * args.timing_steps
             elif name == "jacobi" and w.kind == "uniform" and p.project_mode == 1:
-                bytes_ = 12 * int(info1.active_cells) * n
+                bytes_ = tb[name]
             elif tb.get(name):
                 bytes_ = tb[name]
             if bytes_:
@@ -519,7 +519,7 @@ def main():
         if modelled:
             dom = max(modelled, key=lambda k: modelled[k]["ms_per_step"])
             e = modelled[dom]
-            kname = {"solve_smooth": "k_sv_smooth", "jacobi": "k_jacobi" if w.kind == "dcgrid" else "k_u_jacobi",
+            kname = {"solve_smooth": "k_sv_smooth", "jacobi": "k_jacobi" if w.kind == "dcgrid" else "k_u_sweeps",
                      "advect_velocity": "k_advect_velocity", "advect_density": "k_advect_density",
                      "divergence": "k_divergence", "apply_pressure": "k_apply_pressure"}[dom]
             roof = {"kernel": kname, "bound": "hbm", "achieved": e["algorithmic_GBps"], "peak": HBM_PEAK_GBS,

@@ -756,9 +756,14 @@ struct UniformSim : SimBase {
     const float* in = mode == U_IN_PROLONG ? g.pre + dims[level + 1].off : nullptr;
     float* scratch[2] = {(float*)g.tvel, (float*)g.tvel + n};
     int left = 2 * pairs, chunks = (left + kSweepsPerLaunch - 1) / kSweepsPerLaunch;
-    Pending batch;  // the run of launches is timed as one batch of half-sweeps
+    const uint32_t launches = (uint32_t)chunks;
+    Pending batch;  // the run of launches is timed as one batch
     DCG_TRY(beginTimed(DCG_K_JACOBI, &batch));
     batchK = DCG_K_JACOBI;
+    // bytes of a launch: the divergence and its input read, the last sweep written (and at the end the
+    // one before it)
+    if (batch.k >= 0)
+      timingBytes[DCG_K_JACOBI] += (uint64_t)n * (12 * launches + 4) - (mode == U_IN_ZERO ? n * 4 : n * 7 / 2);
     for (int c = 0; chunks > 0; c++, chunks--) {
       const int k = (left + chunks - 1) / chunks;
       left -= k;
@@ -782,7 +787,7 @@ struct UniformSim : SimBase {
       mode = U_IN_ARRAY;
     }
     batchK = -1;
-    return endTimed(DCG_K_JACOBI, &batch, 2 * pairs);
+    return endTimed(DCG_K_JACOBI, &batch, launches);
   }
   int countStep() override { return DCG_OK; }
   void countHost(uint64_t steps) override { cellStepCount += steps * N; }

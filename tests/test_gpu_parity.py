@@ -344,6 +344,21 @@ def test_uniform_fused_sweeps_bitwise(size, mode, pairs):
     c.close()
 
 
+@pytest.mark.parametrize("size,pairs,launches", [((64, 64, 64), 50, 25), ((40, 33, 21), 1, 1), ((64, 64, 64), 3, 2)])
+def test_uniform_projection_launch_count(size, pairs, launches):
+    """The timing of the half-sweeps counts launches (of up to four of them) and their bytes: 12 per
+    cell, without the first launch's input, which is zero, and with t_pressure written by the last."""
+    p = scenes.reference_params(*size, kind="uniform")
+    p.project_local_pairs = pairs
+    g = dcgrid_amd.Simulation("uniform", size, p)
+    g.set_timing(["jacobi"])
+    g.project_local()
+    ms, n = g.timing()["jacobi"]
+    assert n == launches and ms > 0
+    assert g.timing_bytes()["jacobi"] == 12 * launches * size[0] * size[1] * size[2]
+    g.close()
+
+
 # Samples whose corners all lie in the domain and samples across every face, edge and corner of it, on
 # extents of 1 and 2 (no inner sample), a row of one wavefront and one past it; cells and displacements
 # of several cells in every direction, and (large) back traces from far outside.
