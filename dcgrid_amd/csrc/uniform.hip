@@ -743,6 +743,33 @@ struct UniformSim : SimBase {
   static size_t sweepTiles(const UDims& D, int k, int ty, int tz) {
     return (size_t)sweepColumns(D.w, k) * (size_t)((D.h + ty - 1) / ty) * (size_t)((D.d + tz - 1) / tz);
   }
+  struct SweepTile {
+    int ty, tz;
+  };
+  static SweepTile sweepTile(const UDims& D, int k) {
+    if (sweepTiles(D, k, 4, 4) <= 512) return {4, 4};
+    if (k == 2 && sweepTiles(D, k, 12, 12) >= 1024) return {12, 12};
+    return k == 3 ? SweepTile{10, 10} : SweepTile{8, 8};
+  }
+  // Whether the fused launches of a level's sweeps take less time than one launch per sweep. Their
+  // rows are 64 cells whatever the level's width, so on a thin level most lanes hold nothing, and a tile
+  // of one plane or row is mostly halo. Fitted to 90 projections of domains of 1 to 1024 cells an axis
+  // (each measured both ways, MI355X): a fused launch of k sweeps takes 0.75 k us and 1.05 ps for every
+  // cell of its tiles with their halo, a single sweep 2.25 us and 2.45 ps a cell; the rule is the quotient
+  // of these. 40 sweeps, fused / single: 24 x 256 x 256 247 / 259 us (fused), 16 x 320 x 320 383 / 310,
+  // 8 x 512 x 512 805 / 311, 16 x 1024 x 1024 3170 / 1813, 1 x 1024 x 1024 3012 / 262, 1024 x 1024 x 1
+  // 507 / 262 (single).
+  static bool sweepsFused(const UDims& D, int pairs) {
+    double cells = 0;
+    for (int left = 2 * pairs, chunks = sweepChunks(pairs); chunks > 0; chunks--) {
+      const int k = (left + chunks - 1) / chunks;
+      left -= k;
+      const SweepTile t = sweepTile(D, k);
+      cells += 64.0 * (t.ty + 2 * k) * (t.tz + 2 * k) * (double)sweepTiles(D, k, t.ty, t.tz);
+    }
+    return cells <= 2.0 * pairs * (1.43e6 + 2.33 * (double)ucells(D));
+  }
+  static int sweepChunks(int pairs) { return (2 * pairs + kSweepsPerLaunch - 1) / kSweepsPerLaunch; }
   template <int K, int TY, int TZ>
   void sweepLaunch(const UDims& D, const float* in, int mode, float* out, float* outPrev, float alpha) {
     k_u_sweeps<K, TY, TZ><<<(unsigned)sweepTiles(D, K, TY, TZ), (TY + 2 * K) * 64, 0, stream>>>(
@@ -753,9 +780,10 @@ struct UniformSim : SimBase {
     const size_t n = ucells(D);
     const int scale = 1 << level;
     const float alpha = P.dx * P.dx * (float)scale * (float)scale;  // dx*dx*scale*scale, uniformgrid_fluid.cu:171
+    if (!sweepsFused(D, pairs)) return singleSweeps(level, pairs, mode, alpha);
     const float* in = mode == U_IN_PROLONG ? g.pre + dims[level + 1].off : nullptr;
     float* scratch[2] = {(float*)g.tvel, (float*)g.tvel + n};
-    int left = 2 * pairs, chunks = (left + kSweepsPerLaunch - 1) / kSweepsPerLaunch;
+    int left = 2 * pairs, chunks = sweepChunks(pairs);
     const uint32_t launches = (uint32_t)chunks;
     Pending batch;  // the run of launches is timed as one batch
     DCG_TRY(beginTimed(DCG_K_JACOBI, &batch));
@@ -769,13 +797,13 @@ struct UniformSim : SimBase {
       left -= k;
       float* out = chunks == 1 ? g.pre + D.off : scratch[c & 1];
       float* outPrev = chunks == 1 ? g.tpre + D.off : nullptr;
-      const size_t small = sweepTiles(D, k, 4, 4), wide = sweepTiles(D, k, 12, 12);
-      if (small <= 512) {
+      const SweepTile t = sweepTile(D, k);
+      if (t.ty == 4) {
         if (k == 2) sweepLaunch<2, 4, 4>(D, in, mode, out, outPrev, alpha);
         else if (k == 3) sweepLaunch<3, 4, 4>(D, in, mode, out, outPrev, alpha);
         else sweepLaunch<4, 4, 4>(D, in, mode, out, outPrev, alpha);
       } else if (k == 2) {
-        if (wide >= 1024) sweepLaunch<2, 12, 12>(D, in, mode, out, outPrev, alpha);
+        if (t.ty == 12) sweepLaunch<2, 12, 12>(D, in, mode, out, outPrev, alpha);
         else sweepLaunch<2, 8, 8>(D, in, mode, out, outPrev, alpha);
       } else if (k == 3) {
         sweepLaunch<3, 10, 10>(D, in, mode, out, outPrev, alpha);
@@ -788,6 +816,23 @@ struct UniformSim : SimBase {
     }
     batchK = -1;
     return endTimed(DCG_K_JACOBI, &batch, launches);
+  }
+  // The same with a launch per half-sweep; a zero input is in the pressure array already.
+  int singleSweeps(int level, int pairs, int mode, float alpha) {
+    const UDims& D = dims[level];
+    const size_t n = ucells(D);
+    if (mode == U_IN_PROLONG)
+      DCG_LAUNCH(DCG_K_PROLONGATE, "k_u_prolongate", (k_u_prolongate<<<nblk(n), 256, 0, stream>>>(g.pre, D, dims[level + 1])));
+    Pending batch;  // the run of launches is timed as one batch
+    DCG_TRY(beginTimed(DCG_K_JACOBI, &batch));
+    batchK = DCG_K_JACOBI;
+    if (batch.k >= 0) timingBytes[DCG_K_JACOBI] += (uint64_t)n * 12 * (2 * pairs);
+    for (int i = 0; i < pairs; i++) {
+      DCG_LAUNCH(DCG_K_JACOBI, "k_u_jacobi", (k_u_jacobi<<<nblk(n), 256, 0, stream>>>(g.pre, g.tpre, g.div, D, alpha)));
+      DCG_LAUNCH(DCG_K_JACOBI, "k_u_jacobi", (k_u_jacobi<<<nblk(n), 256, 0, stream>>>(g.tpre, g.pre, g.div, D, alpha)));
+    }
+    batchK = -1;
+    return endTimed(DCG_K_JACOBI, &batch, 2 * pairs);
   }
   int countStep() override { return DCG_OK; }
   void countHost(uint64_t steps) override { cellStepCount += steps * N; }
@@ -848,8 +893,10 @@ struct UniformSim : SimBase {
   // workgroup (k_u_coarse), the others level by level.
   int project() override {
     const int Ls = coarseStart();
-    // level 0 is swept by sweeps(), which writes all of its pressure and t_pressure
-    const bool swept = Ls > 0 && (L > 1 ? P.project_level_pairs : P.project_top_pairs) > 0;
+    // level 0 is swept by sweeps(), which writes all of its pressure and t_pressure (from zero with a launch
+    // per sweep it reads the pressure's zeros)
+    const bool swept =
+        Ls > 0 && (L > 1 ? P.project_level_pairs > 0 : P.project_top_pairs > 0 && sweepsFused(dims[0], P.project_top_pairs));
     DCG_TRY(divergence(!swept));
     for (int l = 1; l < L && l <= Ls; l++) {
       const UDims& D = dims[l];
@@ -873,7 +920,7 @@ struct UniformSim : SimBase {
   }
   // projectLocal(), fluid_simulation_uniform.cu:126-135
   int projectLocal() override {
-    DCG_TRY(divergence(P.project_local_pairs <= 0));
+    DCG_TRY(divergence(P.project_local_pairs <= 0 || !sweepsFused(dims[0], P.project_local_pairs)));
     if (P.project_local_pairs > 0) DCG_TRY(sweeps(0, P.project_local_pairs, U_IN_ZERO));
     return applyPressure();
   }

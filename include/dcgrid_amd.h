@@ -419,7 +419,7 @@ int dcg_timing_get(dcg_sim* s, int32_t kernel, double* total_ms, uint64_t* launc
 /* Algorithmic HBM bytes of the launches timed in class `kernel` since dcg_set_timing, where the
  * library counts them itself (DCG_K_SOLVE_SMOOTH: the correction read and written and the
  * right-hand side read, per cell of the listed blocks; DCG_K_JACOBI on the uniform grid: the pressure
- * read and written and the divergence read, per launch of up to four half-sweeps; 0 for the other
+ * read and written and the divergence read, per launch; 0 for the other
  * classes, whose work is a function of the block loads the caller can read). */
 int dcg_timing_bytes(dcg_sim* s, int32_t kernel, uint64_t* bytes);
 
@@ -428,8 +428,8 @@ enum {
   DCG_K_ADVECT_VELOCITY = 0,
   DCG_K_ADVECT_DENSITY = 1,
   DCG_K_DIVERGENCE = 2,
-  DCG_K_JACOBI = 3,     /* on the uniform grid a launch runs up to four half-sweeps, and the first of */
-  DCG_K_PROLONGATE = 4, /* a level prolongs its input itself, so that class 4 has no launch there */
+  DCG_K_JACOBI = 3,     /* on the uniform grid a launch runs up to four half-sweeps, and the first of a */
+  DCG_K_PROLONGATE = 4, /* level prolongs its input itself (thin domains: one each, and a prolongation) */
   DCG_K_APPLY_PRESSURE = 5,
   DCG_K_RESTRICT = 6,
   DCG_K_TOPOLOGY = 7,

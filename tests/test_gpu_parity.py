@@ -313,7 +313,10 @@ SWEEP_CASES = [((1, 1, 1), "local", 1), ((2, 3, 1), "local", 2), ((64, 5, 9), "l
                ((120, 9, 10), "local", 2), ((121, 12, 13), "local", 7), ((176, 33, 21), "local", 2),
                ((63, 100, 104), "local", 2), ((70, 100, 104), "local", 3), ((64, 100, 104), "local", 1),
                ((64, 384, 384), "multilevel", 1), ((128, 64, 96), "multilevel", 1), ((64, 96, 128), "multilevel", 3),
-               ((34, 38, 46), "multilevel", 2)]
+               ((34, 38, 46), "multilevel", 2),
+               # thin domains, with a launch per sweep: along every axis, from zero and from a coarser level
+               ((4, 4, 4096), "local", 2), ((1, 512, 512), "local", 1), ((640, 640, 1), "local", 3),
+               ((640, 640, 1), "multilevel", 1), ((8, 256, 256), "multilevel", 1), ((8, 256, 256), "multilevel", 2)]
 
 
 @pytest.mark.parametrize("size,mode,pairs", SWEEP_CASES)
@@ -344,10 +347,12 @@ def test_uniform_fused_sweeps_bitwise(size, mode, pairs):
     c.close()
 
 
-@pytest.mark.parametrize("size,pairs,launches", [((64, 64, 64), 50, 25), ((40, 33, 21), 1, 1), ((64, 64, 64), 3, 2)])
+@pytest.mark.parametrize("size,pairs,launches", [((64, 64, 64), 50, 25), ((40, 33, 21), 1, 1), ((64, 64, 64), 3, 2),
+                                                 ((1, 512, 512), 5, 10), ((512, 512, 1), 8, 16), ((16, 320, 320), 1, 2)])
 def test_uniform_projection_launch_count(size, pairs, launches):
-    """The timing of the half-sweeps counts launches (of up to four of them) and their bytes: 12 per
-    cell, without the first launch's input, which is zero, and with t_pressure written by the last."""
+    """The timing of the half-sweeps counts launches and their bytes, 12 per cell: of up to four half-sweeps
+    (without the first launch's input, which is zero, and with t_pressure written by the last), and of one
+    each on thin domains, which fill too few of the fused launch's lanes."""
     p = scenes.reference_params(*size, kind="uniform")
     p.project_local_pairs = pairs
     g = dcgrid_amd.Simulation("uniform", size, p)
