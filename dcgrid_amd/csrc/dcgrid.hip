@@ -27,7 +27,9 @@ namespace dcg {
 // block's apron around the position in the block's level.
 template <int BW, class G>
 struct DCMarchSampler {
+  static constexpr bool kDense = false;  // cells by index, without a walk to the sample's block
   G g;
+  template <int GL>
   __device__ void sample(const dcg_params& P, int precise, float3 pos, MarchAux& a) const {
     constexpr int BB = Geo<BW>::BB, BV = Geo<BW>::BV;
     const int ix = clampi((int)floorf(pos.x), 0, g.gx - 1);
@@ -52,7 +54,10 @@ struct DCMarchSampler {
     const int ai = clampi((int)(xf + 1.f - (float)bp.x), 0, BW);
     const int aj = clampi((int)(yf + 1.f - (float)bp.y), 0, BW);
     const int ak = clampi((int)(zf + 1.f - (float)bp.z), 0, BW);
-    if (ai > 0 && ai < BW && aj > 0 && aj < BW && ak > 0 && ak < BW) {  // all corners in the block
+    if (GL == 1) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) a.cell[k] = apronCell<BW>(g, b, ai + ((k >> 2) & 1), aj + ((k >> 1) & 1), ak + (k & 1));
+    } else if (ai > 0 && ai < BW && aj > 0 && aj < BW && ak > 0 && ak < BW) {  // all corners in the block
 #pragma unroll
       for (int k = 0; k < 8; k++)
         a.cell[k] = b * BV + loc<BB>(ai - 1 + ((k >> 2) & 1), aj - 1 + ((k >> 1) & 1), ak - 1 + (k & 1));
@@ -1243,7 +1248,9 @@ struct DCGridSim : SimBase {
   }
   int render(const dcg_render_params& r, float* rgba) override {
     DCMarchSampler<BW, DGT<SF>> smp{g};
-    DCG_LAUNCH(DCG_K_OTHER, "k_render", (launchRender(smp, P, r, (float4*)rgba, stream)));
+    const MarchRoute route = marchRoute<decltype(smp)>(P, r);
+    if (route.begin) DCG_LAUNCH(DCG_K_OTHER, "k_render_begin", (launchRenderBegin(P, r, (float4*)rgba, stream)));
+    DCG_LAUNCH(DCG_K_OTHER, "k_render", (launchRender(smp, route, P, r, (float4*)rgba, stream)));
     return DCG_OK;
   }
 

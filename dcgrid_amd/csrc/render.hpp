@@ -2,7 +2,7 @@
 // (src/fluid_simulation.h:19) for both grids, following src/raymarching.cuh:63-275 with the
 // samplers of src/dcgrid/dcgrid_rendering.cu:6-64 and src/uniformgrid/uniformgrid_rendering.cu:5-47.
 //
-// Sixteen lanes per ray (MarchGroup). Every float operation is written out in the order of the
+// One, 4 or 16 lanes per ray (MarchGroup, marchRoute). Every float operation is written out in the order of the
 // reference's helper_math expressions, with correctly rounded division and square root and the
 // library's own deterministic exp, so the image equals the oracle's restatement bit for bit.
 // Deliberate differences: normalize divides by the length (helper_math multiplies by rsqrtf); the
@@ -115,7 +115,8 @@ __device__ __forceinline__ float3 sceneNormal(const dcg_params& P, float3 p) {
 // DPP row, or a quad of 4) take a ray together: each lane samples its own step of the next GL, and the sums that have to run
 // in the ray's order (positions, optical depth, compositing) are formed by every lane alike from
 // its neighbours' values, in the same order and with the same float operations as by one thread.
-// GL = 1 is the plain loop, for the debug slices (one sample per ray, nothing to share).
+// GL = 1 is the plain loop, for images that fill the chip by themselves and the debug slices (marchRoute
+// draws the line).
 // Measured (MI355X, one thread per ray -> 16 lanes, 256 x 256): plume on the 256^3 grid 34 -> 3.0 ms,
 // on the 512^3 grid 51 -> 3.7 ms, 4^3 blocks with a solid sphere 35 -> 3.2 ms, dense 64^3 grid
 // 1.2 -> 0.30 ms, terrain 2.4 -> 0.72 ms.
@@ -179,25 +180,31 @@ __device__ __forceinline__ float fluidLight(const S& smp, const dcg_params& P, c
   }
   const float step = fmaxf(dFar / 100.f, 1e-1f);
   const float3 ds = v3mul(sun, step);
+  float density = 0.f;
+  if constexpr (GL == 1) {
+    for (float d = step; d < dFar && density < 5.f; d = d + step) {
+      pos = v3add(pos, ds);
+      smp.template sample<GL>(P, R.precise, pos, aux);
+      density = density + aux.density * P.dx * step;
+    }
+    return lt * marchExp(-density);
+  }
   // the lane's step of the first round: distance and position after lane() + 1 steps
   const int lane = M::lane();
   float d = step;
   pos = v3add(pos, ds);
-  if (GL > 1) {
 #pragma unroll
-    for (int j = 1; j < GL; j++) {
-      const float3 q = v3add(pos, ds);
-      if (lane >= j) {
-        pos = q;
-        d = d + step;
-      }
+  for (int j = 1; j < GL; j++) {
+    const float3 q = v3add(pos, ds);
+    if (lane >= j) {
+      pos = q;
+      d = d + step;
     }
   }
-  float density = 0.f;
   for (;;) {
     float c = 0.f;  // adds nothing for a lane past the end
     if (d < dFar) {
-      smp.sample(P, R.precise, pos, aux);
+      smp.template sample<GL>(P, R.precise, pos, aux);
       c = aux.density * P.dx * step;
     }
     M::each([&](auto J) {
@@ -261,6 +268,9 @@ __device__ __forceinline__ MarchSolid marchSolid(const dcg_params& P, const dcg_
   return m;
 }
 
+// Where a ray that enters the domain at dNear begins its march (Z_NEAR 10).
+__device__ __forceinline__ float marchStart(float dNear) { return fmaxf(0.f, fmaxf(dNear, 10.f)); }
+
 // raymarch (src/raymarching.cuh:123-275); returns (color, alpha), the same in the whole group.
 template <int GL, class S>
 __device__ __forceinline__ float4 rayMarch(const S& smp, const dcg_params& P, const dcg_render_params& R, float3 origin,
@@ -284,11 +294,26 @@ __device__ __forceinline__ float4 rayMarch(const S& smp, const dcg_params& P, co
   if (R.channel == DCG_RENDER_FLUID) {
     float dNear, dFar;
     if (rayDomain(P, dNear, dFar, origin, dirInv)) {
-      float dCurrent = fmaxf(0.f, fmaxf(dNear, 10.f));  // Z_NEAR
+      float dCurrent = marchStart(dNear);
       const float dMax = fminf(dFar, dSolid);
-      const int lane = M::lane();
+      auto shade = [&](float light, float sa) {
+        light = R.ambient + light * ambientInv;
+        marchMix(make_float3(light * R.smoke_color[0], light * R.smoke_color[1], light * R.smoke_color[2]), sa, color, alpha);
+      };
       auto next = [&](float d) { return fminf(fmaxf(d * 1.f, d + .5f), dMax); };  // STEP_MULTIPLIER 1
-      while (dCurrent < dMax && alpha <= .99f) {
+      float3 pos = v3add(origin, v3mul(dir, dCurrent));
+      while (GL == 1 && dCurrent < dMax && alpha <= .99f) {
+        const float3 prev = pos;
+        dCurrent = next(dCurrent);
+        pos = v3add(origin, v3mul(dir, dCurrent));
+        const float3 mid = v3mul(v3add(prev, pos), .5f);
+        smp.template sample<GL>(P, R.precise, mid, aux);
+        if (!(aux.density > 1e-6f)) continue;
+        const float sa = densityToAlpha(P, aux.density, v3len(v3sub(pos, prev)));
+        shade(R.shadows ? fluidLight<GL>(smp, P, R, mid, sceneLight(P, R, mid, sun), aux, sun, sunInv) : 1.f, sa);
+      }
+      const int lane = M::lane();
+      while (GL > 1 && dCurrent < dMax && alpha <= .99f) {
         // the next GL steps: lane k goes from the distance after k of them to the one after k + 1
         float d0 = dCurrent;
 #pragma unroll
@@ -299,9 +324,10 @@ __device__ __forceinline__ float4 rayMarch(const S& smp, const dcg_params& P, co
         float density = 0.f, sa = 0.f, lt = 1.f;
         float3 mid = make_float3(0.f, 0.f, 0.f);
         if (d0 < dMax) {
-          const float3 prev = v3add(origin, v3mul(dir, d0)), pos = v3add(origin, v3mul(dir, next(d0)));
+          const float3 prev = v3add(origin, v3mul(dir, d0));
+          pos = v3add(origin, v3mul(dir, next(d0)));
           mid = v3mul(v3add(prev, pos), .5f);
-          smp.sample(P, R.precise, mid, aux);
+          smp.template sample<GL>(P, R.precise, mid, aux);
           density = aux.density;
           if (density > 1e-6f) {
             sa = densityToAlpha(P, density, v3len(v3sub(pos, prev)));
@@ -312,14 +338,12 @@ __device__ __forceinline__ float4 rayMarch(const S& smp, const dcg_params& P, co
         for (uint32_t todo = M::ballot(density > 1e-6f); todo != 0 && alpha <= .99f; todo &= todo - 1) {
           const int j = __ffs(todo) - 1;
           const float saj = M::at(sa, j);
-          illum = 1.f;
+          float light = 1.f;
           if (R.shadows) {
             const float3 mj = make_float3(M::at(mid.x, j), M::at(mid.y, j), M::at(mid.z, j));
-            illum = illum * fluidLight<GL>(smp, P, R, mj, M::at(lt, j), aux, sun, sunInv);
+            light = fluidLight<GL>(smp, P, R, mj, M::at(lt, j), aux, sun, sunInv);
           }
-          illum = R.ambient + illum * ambientInv;
-          marchMix(make_float3(illum * R.smoke_color[0], illum * R.smoke_color[1], illum * R.smoke_color[2]), saj, color,
-                   alpha);
+          shade(light, saj);
         }
       }
     }
@@ -345,7 +369,7 @@ __device__ __forceinline__ float4 rayMarch(const S& smp, const dcg_params& P, co
   }
   if (what == MARCH_DEBUG) {
     pos.z = sliceZ;
-    smp.sample(P, R.precise, pos, aux);
+    smp.template sample<GL>(P, R.precise, pos, aux);
     if (R.channel == DCG_RENDER_DENSITY) {
       const float v = aux.density * 1e2f;
       marchMix(make_float3(v, 0.f, 0.f), 1.f, color, alpha);
@@ -377,21 +401,46 @@ __device__ __forceinline__ float3 marchOrigin(const dcg_params& P, const dcg_ren
   return make_float3(R.eye_origin[0] * P.rdx, R.eye_origin[1] * P.rdx, R.eye_origin[2] * P.rdx);
 }
 
-// What every pixel's ray meets behind the fluid, left in the image for k_render (one ray per
-// pixel): d, what and lt in x, y and z.
-static __global__ void __launch_bounds__(256) k_render_solids(dcg_params P, dcg_render_params R, float4* __restrict__ out) {
+// For rays that meet no fluid.
+struct NoFluid {
+  template <int GL>
+  __device__ void sample(const dcg_params&, int, float3, MarchAux&) const {}
+  __device__ float3 velocity(const MarchAux&) const { return make_float3(0.f, 0.f, 0.f); }
+  __device__ float fluidity(const MarchAux&) const { return 0.f; }
+};
+// A thread per ray before the rays are marched by several lanes each (one ray per pixel, the marched
+// channel): a ray that has no fluid to cross and whose background no fluid can shade is finished here;
+// of the others the image takes what they meet behind the fluid: d, what, lt, and kMarchOpen (a NaN that
+// no arithmetic makes) where a finished pixel has its opacity.
+static constexpr int kMarchOpen = 0x7FC5A5A5;
+static __global__ void __launch_bounds__(256) k_render_begin(dcg_params P, dcg_render_params R, float4* __restrict__ out) {
   const int x = blockIdx.x * 16 + (int)(threadIdx.x % 16), y = blockIdx.y * 16 + (int)(threadIdx.x / 16);
   if (x >= R.width || y >= R.height) return;
   const float3 sun = make_float3(R.sun_dir[0], R.sun_dir[1], R.sun_dir[2]);
-  const MarchSolid m = marchSolid(P, R, marchOrigin(P, R), marchDirection(R, x, y, 0.f, 0.f), sun);
-  out[(size_t)y * R.width + x] = make_float4(m.d, __int_as_float(m.what), m.lt, 0.f);
+  const float3 origin = marchOrigin(P, R), dir = marchDirection(R, x, y, 0.f, 0.f);
+  const MarchSolid m = marchSolid(P, R, origin, dir, sun);
+  float dNear, dFar;
+  bool open = rayDomain(P, dNear, dFar, origin, make_float3(1.f / dir.x, 1.f / dir.y, 1.f / dir.z)) &&
+              marchStart(dNear) < fminf(dFar, m.d);
+  if (!open && R.shadows && m.what != MARCH_NONE && m.lt != 0.f) {
+    float3 pos = v3add(origin, v3mul(dir, m.d));
+    if (m.what == MARCH_FLOOR) pos.y = 0.f;
+    open = rayDomain(P, dNear, dFar, pos, make_float3(1.f / sun.x, 1.f / sun.y, 1.f / sun.z));
+  }
+  float4 c = make_float4(m.d, __int_as_float(m.what), m.lt, __int_as_float(kMarchOpen));
+  if (!open) {
+    c = rayMarch<1>(NoFluid{}, P, R, origin, dir, sun, m);
+    c = make_float4(0.f + c.x, 0.f + c.y, 0.f + c.z, 0.f + c.w);  // k_render's sum over one ray
+  }
+  out[(size_t)y * R.width + x] = c;
 }
 
 // k_dcgrid_render / k_uniform_render: per pixel, aa_samples^2 rays averaged. A workgroup takes a
-// tile of T x T pixels with GL lanes per ray. SOLIDS: the pixel's entry of the image holds what its
-// one ray meets behind the fluid (k_render_solids).
-template <int GL, int T, bool SOLIDS, class S>
-__global__ void __launch_bounds__(T* T* GL) k_render(S smp, dcg_params P, dcg_render_params R, float4* __restrict__ out) {
+// tile of T x T pixels with GL lanes per ray. BEGUN: the pixel's entry of the image comes from
+// k_render_begin. One lane per ray runs on images that fill the chip: four wavefronts a SIMD (at most 128
+// VGPRs) instead of three take 1.05-1.16x off them.
+template <int GL, int T, bool BEGUN, class S>
+__global__ void __launch_bounds__(T* T* GL, GL == 1 ? 4 : 1) k_render(S smp, dcg_params P, dcg_render_params R, float4* __restrict__ out) {
   const int ray = (int)(threadIdx.x / GL);
   const int x = blockIdx.x * T + ray % T, y = blockIdx.y * T + ray / T;
   if (x >= R.width || y >= R.height) return;
@@ -403,8 +452,9 @@ __global__ void __launch_bounds__(T* T* GL) k_render(S smp, dcg_params P, dcg_re
     for (float dy = 0.f; dy < 1.f; dy = dy + step) {
       const float3 dir = marchDirection(R, x, y, dx, dy);
       MarchSolid solid;
-      if (SOLIDS) {
+      if (BEGUN) {
         const float4 m = out[(size_t)y * R.width + x];
+        if (__float_as_int(m.w) != kMarchOpen) return;  // finished there
         solid = MarchSolid{m.x, __float_as_int(m.y), m.z};
       } else {
         solid = marchSolid(P, R, origin, dir, sun);
@@ -417,33 +467,64 @@ __global__ void __launch_bounds__(T* T* GL) k_render(S smp, dcg_params P, dcg_re
   out[(size_t)y * R.width + x] = make_float4(acc.x * w, acc.y * w, acc.z * w, acc.w * w);
 }
 
-// The launches of a render. The marched channel takes 16 lanes per ray up to 512 K pixels and 4 above,
-// the debug slices one thread. The ray's fixed cost is paid by every lane, so once the image alone
-// fills the chip fewer lanes win (1920 x 1080, 16 -> 4 lanes: plume 24.1 -> 16.5 ms, dense grid 2.9 ->
-// 1.1 ms, terrain 15.2 -> 11.1 ms; at 512 x 512 16 lanes are the faster, 8.5 -> 4.4 ms on the plume).
-// A solid scene's sphere traces (up to 200 scene distances a ray, each a 5-octave noise with a
-// terrain) cannot be shared by a ray's lanes: a pass of its own takes them a thread per ray, and
-// leaves its results in the image, which holds them for one ray per pixel; with several the whole
-// march runs a thread per ray (a trace by 16 lanes alike takes 16 times the instructions: a terrain
-// image of 1024 x 768 took 17.8 ms with the traces in the march's workgroups, 4.4 ms this way).
+// The launches of a render: lanes per ray, and whether k_render_begin goes first.
+//
+// The ray's fixed cost and the sums in its order are paid by every lane, so lanes win while the image
+// has too few rays for the chip (2^18 threads of this kernel are resident) or rays of very unequal
+// length (shadow marches), and lose where a thread per ray fills it. The lines lie where no scene with fluid
+// in view is slower than with one lane by more than the noise (MI355X; DCGrid scenes of 128^3 to 512^3 cells,
+// plume and sphere, and dense grids, 64^3 with a plume and 200^3 filled with fluid; gain over one lane):
+//   DCGrid, shadows      724 x 724: 16 lanes 5.1-8.3x, 4 lanes 3.0-4.1x; 1920 x 1080: 4 lanes 1.5-2.1x, 16
+//                        1.0-2.0x; 3840 x 2160: 4 lanes 0.8-1.1x
+//   DCGrid, no shadows   512 x 512: 16 and 4 lanes 1.6-2.5x; 1024 x 768: 4 lanes 1.05-1.45x; 1920 x 1080: 0.8-1.0x
+//   dense, shadows       256 x 256: 16 lanes 4.2-4.7x; 512 x 512: 4 lanes 1.6-2.6x, 16 1.3-3.2x; 1024 x 768: 4 lanes
+//                        1.3-1.9x, 16 0.75-1.4x; 1920 x 1080: 4 lanes 0.8-1.2x
+//   dense, no shadows    128 x 128: 16 lanes 2.8-3.8x; 256 x 256: 4 lanes 2.0x, 16 1.3-1.8x; 512 x 512: 4 lanes
+//                        1.0-1.2x; 724 x 724: 0.9-1.0x
+// A solid scene's traces (up to 200 scene distances a ray) cannot be shared by a ray's lanes and are left to
+// k_render_begin, a thread per ray. With a terrain, each distance a 5-octave noise, they are most of
+// the image and no longer hidden beside the march: 16 lanes up to 512 x 512 (there 1.2-1.9x; 0.95 with coarse
+// samples or no fluid in view), one above (0.8-1.1 with 16), and one with several rays per pixel, which the
+// image cannot hold (16 lanes 0.1-0.5x). The finishing of rays that meet no fluid is worth a launch of its own from
+// 2^16 pixels on; an image of nothing but such rays pays for it (1920 x 1080: 21 -> 65 us).
+struct MarchRoute {
+  int lanes;
+  bool begin;
+};
 template <class S>
-void launchRender(const S& smp, const dcg_params& P, const dcg_render_params& R, float4* out, hipStream_t stream) {
-  auto grid = [&](int t) { return dim3((unsigned)((R.width + t - 1) / t), (unsigned)((R.height + t - 1) / t)); };
-  const bool scene = R.solids && P.enable_additional_solids;
-  const bool wide = (size_t)R.width * R.height <= (size_t)512 * 1024;
-  if (R.channel != DCG_RENDER_FLUID || (scene && R.aa_samples > 1.f)) {
-    k_render<1, 16, false><<<grid(16), 256, 0, stream>>>(smp, P, R, out);
-  } else if (scene) {
-    k_render_solids<<<grid(16), 256, 0, stream>>>(P, R, out);
-    if (wide)
-      k_render<16, 4, true><<<grid(4), 256, 0, stream>>>(smp, P, R, out);
-    else
-      k_render<4, 8, true><<<grid(8), 256, 0, stream>>>(smp, P, R, out);
-  } else if (wide) {
-    k_render<16, 4, false><<<grid(4), 256, 0, stream>>>(smp, P, R, out);
+MarchRoute marchRoute(const dcg_params& P, const dcg_render_params& R) {
+  if (R.channel != DCG_RENDER_FLUID) return {1, false};  // one sample per ray
+  const size_t pixels = (size_t)R.width * R.height;
+  const bool scene = R.solids && P.enable_additional_solids, single = R.aa_samples <= 1.f;
+  int lanes;
+  if (scene && P.solid_mode == DCG_SOLID_TERRAIN) {
+    lanes = single && pixels <= (size_t)1 << 18 ? 16 : 1;
   } else {
-    k_render<4, 8, false><<<grid(8), 256, 0, stream>>>(smp, P, R, out);
+    const int most16 = S::kDense ? (R.shadows ? 17 : 15) : (R.shadows ? 19 : 18);  // log2 of the pixels
+    const int most4 = S::kDense ? (R.shadows ? 20 : 18) : (R.shadows ? 21 : 20);
+    lanes = pixels <= (size_t)1 << most16 ? 16 : pixels <= (size_t)1 << most4 ? 4 : 1;
   }
+  return {lanes, lanes > 1 && single && (scene || pixels > (size_t)1 << 16)};
+}
+static inline dim3 marchGrid(const dcg_render_params& R, int tile) {
+  return dim3((unsigned)((R.width + tile - 1) / tile), (unsigned)((R.height + tile - 1) / tile));
+}
+static inline void launchRenderBegin(const dcg_params& P, const dcg_render_params& R, float4* out, hipStream_t stream) {
+  k_render_begin<<<marchGrid(R, 16), 256, 0, stream>>>(P, R, out);
+}
+template <class S>
+void launchRender(const S& smp, MarchRoute route, const dcg_params& P, const dcg_render_params& R, float4* out,
+                  hipStream_t stream) {
+  if (route.lanes == 1)
+    k_render<1, 16, false><<<marchGrid(R, 16), 256, 0, stream>>>(smp, P, R, out);
+  else if (route.lanes == 4 && route.begin)
+    k_render<4, 8, true><<<marchGrid(R, 8), 256, 0, stream>>>(smp, P, R, out);
+  else if (route.lanes == 4)
+    k_render<4, 8, false><<<marchGrid(R, 8), 256, 0, stream>>>(smp, P, R, out);
+  else if (route.begin)
+    k_render<16, 4, true><<<marchGrid(R, 4), 256, 0, stream>>>(smp, P, R, out);
+  else
+    k_render<16, 4, false><<<marchGrid(R, 4), 256, 0, stream>>>(smp, P, R, out);
 }
 
 }  // namespace dcg

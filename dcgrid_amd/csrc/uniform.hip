@@ -32,7 +32,9 @@ struct UGrid {
 // coarse = the cell of the truncated position, precise = trilinear with the reference's
 // edge handling (the lower corner clamped, the upper one repeated at the far faces).
 struct UMarchSampler {
+  static constexpr bool kDense = true;  // cells by index, without a walk to the sample's block
   UGrid g;
+  template <int GL>
   __device__ void sample(const dcg_params& P, int precise, float3 pos, MarchAux& a) const;
   __device__ float3 velocity(const MarchAux& a) const { return marchInterp3(g.vel, a); }
   __device__ float fluidity(const MarchAux& a) const { return marchInterp(g.flu, a); }
@@ -46,6 +48,7 @@ struct UDims {
 __device__ __forceinline__ size_t uidx(const UGrid& g, int x, int y, int z) {
   return ((size_t)z * g.gy + y) * g.gx + x;
 }
+template <int GL>
 __device__ void UMarchSampler::sample(const dcg_params& P, int precise, float3 pos, MarchAux& a) const {
   if (!precise) {
     const int ix = clampi((int)pos.x, 0, g.gx - 1), iy = clampi((int)pos.y, 0, g.gy - 1);
@@ -967,7 +970,9 @@ struct UniformSim : SimBase {
   }
   int render(const dcg_render_params& r, float* rgba) override {
     UMarchSampler smp{g};
-    DCG_LAUNCH(DCG_K_OTHER, "k_render", (launchRender(smp, P, r, (float4*)rgba, stream)));
+    const MarchRoute route = marchRoute<decltype(smp)>(P, r);
+    if (route.begin) DCG_LAUNCH(DCG_K_OTHER, "k_render_begin", (launchRenderBegin(P, r, (float4*)rgba, stream)));
+    DCG_LAUNCH(DCG_K_OTHER, "k_render", (launchRender(smp, route, P, r, (float4*)rgba, stream)));
     return DCG_OK;
   }
 

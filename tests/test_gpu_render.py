@@ -44,6 +44,10 @@ def workload(name):
         p = w.params.copy()
         p.enable_additional_solids = 1
         return w.kind, w.size, p, None
+    if name == "ref48_uniform_solids":  # the sphere and the inlet's fluid in view
+        p = scenes.reference_params(48, kind="uniform")
+        p.enable_additional_solids = 1
+        return "uniform", (48, 48, 48), p, None
     raise KeyError(name)
 
 
@@ -132,5 +136,55 @@ def test_render_lanes_per_ray(name, size):
         b = g.render(half)
         assert size[0] * size[1] > 512 * 1024 >= half.width * half.height
         assert same(a[1:-1], b), (name, size)
+    g.close()
+    c.close()
+
+
+# One pixel row past each line of the rule that gives a ray its lanes, and one before: (scene, image, shadows,
+# launches on either side). Two launches where rays that meet no fluid are finished by a launch of
+# their own (several lanes a ray and more than 2^16 pixels, or a solid scene), one otherwise.
+LANE_LINES = [("cfg1_64", (1449, 1448), 1, (1, 2)), ("cfg1_64", (513, 512), 0, (2, 2)), ("cfg1_64", (1025, 1024), 0, (1, 2)),
+              ("cfg0_32", (513, 256), 1, (2, 2)), ("cfg0_32", (1025, 1024), 1, (1, 2)), ("cfg0_32", (257, 128), 0, (1, 1)),
+              ("cfg0_32", (513, 512), 0, (1, 2)), ("cfg0_32", (257, 256), 1, (2, 1)), ("ref48_uniform_solids", (33, 32), 1, (2, 2)),
+              ("cfg4_128", (513, 512), 1, (1, 2))]
+
+
+@pytest.mark.parametrize("name,size,shadows,launches", LANE_LINES)
+def test_render_lane_lines(name, size, shadows, launches):
+    """The image does not depend on the lanes per ray: the inner rows on one side of a line equal the
+    same rays on the other side (the pixel pitch follows the larger side). A sky view has rays that pass
+    the domain by."""
+    kind, shape, p, b = workload("cfg0_32_solids" if name == "cfg0_32" else name)
+    p = p.copy()
+    if name == "cfg0_32":
+        p.enable_additional_solids = 0
+    g = dcgrid_amd.Simulation(kind, shape, p, b)
+    if not name.startswith("ref"):
+        g.seed_scene()
+    g.step(3)
+    r = g.default_render_params()
+    r.shadows = shadows
+    for up in (-.2, .3):
+        r.eye_dir[1], r.eye_dir[2] = up, float(np.sqrt(1 - up * up))
+        images = []
+        for rows, n in zip((size[1], size[1] - 2), launches):
+            r.width, r.height = size[0], rows
+            g.set_timing(["other"])
+            images.append(g.render(r))
+            assert g.timing()["other"][1] == n, (name, size, rows)
+        assert same(images[0][1:-1], images[1]), (name, size, up)
+    g.close()
+
+
+@pytest.mark.parametrize("name", ["cfg1_64", "ref48_uniform_solids", "ref64_bw4_solids", "cfg4_128"])
+def test_render_several_rays_with_shadows(name):
+    """Four rays per pixel with shadow marches equal the oracle's: 16 lanes a ray (without and with a solid
+    sphere, whose traces the lanes repeat) and one (terrain)."""
+    g, c = pair(name)
+    r = g.default_render_params()
+    r.width, r.height, r.aa_samples, r.shadows = 23, 14, 2.0, 1
+    a, b = g.render(r), c.render(r)
+    assert same(a, b), name
+    assert len(np.unique(a.reshape(-1, 4), axis=0)) > 2
     g.close()
     c.close()
