@@ -70,7 +70,8 @@ def same(a, b):
     return np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-@pytest.mark.parametrize("name", ["cfg1_64", "ref64_bw4_solids", "cfg4_128", "cfg1_64_fp16", "cfg0_32_solids"])
+@pytest.mark.parametrize("name", ["cfg1_64", "ref64_bw4_solids", "cfg4_128", "cfg1_64_fp16", "cfg0_32_solids",
+                                  "ref48_uniform_solids"])
 def test_render_bitwise_vs_oracle(name):
     say(f"[case] render {name}")
     g, c = pair(name)
@@ -121,9 +122,9 @@ def test_device_pointer_and_checks():
                                        ("cfg0_32_solids", (1025, 512))])
 def test_render_lanes_per_ray(name, size):
     """The marched channel at the edges of its launch shapes: partial tiles (an image smaller than a
-    tile, one past it), and one pixel row past the 512 K pixels from which 4 lanes take a ray instead
-    of 16. The small images equal the oracle's; the large one's inner rows equal those of an image
-    two rows lower, which takes 16 lanes."""
+    tile, one past it), and one pixel row past the 512 K pixels from which 4 lanes take a DCGrid's ray
+    instead of 16 (on the dense grid, where the camera is inside the solid, both images take 4). The small
+    images equal the oracle's; the large one's inner rows equal those of an image two rows lower."""
     g, c = pair(name)
     r = g.default_render_params()
     r.width, r.height = size

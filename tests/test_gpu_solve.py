@@ -188,20 +188,38 @@ def test_precision_variants():
     assert max(res[SOLVE_FP32][0]["rel_residual"]) > 1e-8 or e_32 <= 1e-5
 
 
-# Dense grids around the direct solve's tiles: axes below and past multiples of 32 (padded transform
-# halves), of one block, with partial column tiles (z frequencies, block columns), BW 4 and 8, the
-# longest axis of the 64-line tiles (256), past it (320), of the 32-line tiles (512) and of all (1024).
-DIRECT_CASES = [((64, 96, 160), 8, 3), ((48, 16, 80), 8, 2), ((8, 8, 8), 8, 1), ((24, 8, 40), 8, 1), ((24, 40, 56), 4, 2),
-                ((16, 16, 16), 4, 3), ((20, 4, 12), 4, 1), ((256, 16, 32), 8, 2), ((16, 320, 32), 8, 2),
-                ((16, 32, 512), 8, 2), ((512, 16, 16), 8, 2), ((1024, 16, 16), 8, 2)]
+# Dense grids around the direct solve's tiles, with the lines of the finest level's x, y and z passes: axes
+# below and past multiples of 32 (padded transform halves), of one block, BW 4 and 8; the longest axes of the
+# 32-line tiles (512) and of the 16-line ones (1024) along x, y and z (where 16 lines are part of a
+# block column); 64-line tiles of 16 and of several matrix tiles, up to the longest (256), with padded
+# halves (136, 132), and for BW 4 with four block columns a tile, the last one partial in every pass.
+DIRECT_CASES = [((64, 96, 160), 8, 3, (32, 32, 32)), ((48, 16, 80), 8, 2, (32, 32, 32)), ((8, 8, 8), 8, 1, (32, 32, 32)),
+                ((24, 8, 40), 8, 1, (32, 32, 32)), ((24, 40, 56), 4, 2, (32, 32, 32)), ((16, 16, 16), 4, 3, (32, 32, 32)),
+                ((20, 4, 12), 4, 1, (32, 32, 32)), ((256, 16, 32), 8, 2, (32, 32, 32)), ((16, 320, 32), 8, 2, (32, 32, 32)),
+                ((16, 32, 512), 8, 2, (64, 32, 32)), ((512, 16, 16), 8, 2, (32, 32, 32)),
+                ((1024, 16, 16), 8, 2, (16, 64, 64)), ((16, 1024, 16), 8, 1, (64, 16, 64)),
+                ((16, 16, 1024), 8, 1, (64, 64, 16)), ((8, 12, 520), 4, 1, (32, 32, 16)),
+                ((256, 128, 256), 8, 2, (64, 64, 64)), ((136, 136, 136), 8, 1, (64, 64, 64)),
+                ((132, 132, 132), 4, 1, (64, 64, 64))]
 
 
-@pytest.mark.parametrize("size,bw,levels", DIRECT_CASES)
-def test_dense_levels_against_cosine_transform(size, bw, levels):
+def direct_lines(size, bw):
+    """The lines of a tile in the x, y and z passes by the direct solve's rule: 16 beyond 512 cells of the
+    axis, 64 where the axis has at most 256 and the pass at least 256 tiles of them, else 32."""
+    up = lambda a, b: -(-a // b)  # noqa: E731
+    nx, ny, nz = size
+    tiles = (up(ny * nz, 64), nx // bw * up(nz, 64 // bw), up(nx * ny, 64))
+    return tuple(16 if n > 512 else 64 if n <= 256 and t >= 256 else 32 for n, t in zip(size, tiles))
+
+
+@pytest.mark.parametrize("size,bw,levels,lines", DIRECT_CASES)
+def test_dense_levels_against_cosine_transform(size, bw, levels, lines):
     """Every level of a fully dense grid is a box with Neumann walls: its pressure is the zero-mean
     solution of scipy's DCT-II in 64 bits, to the rounding of the stored FP32 pressure (1e-7 covers
-    its 6e-8); throughout FP32 to that rounding times the longest axis' condition (n / pi)^2."""
+    its 6e-8); throughout FP32 to the residual's rounding, which the smoothest mode of the longest axis
+    (one of all cells) amplifies by (n / pi)^2: 6e-8 (20 + 40 (n / pi)^2 / sqrt(cells))."""
     from scipy.fft import dctn, idctn
+    assert direct_lines(size, bw) == lines
     p = scenes.reference_params(*size)
     p.dt, p.dx, p.rdx = 0.1, 1.0, 1.0
     p.emission_radius = 0.0
@@ -242,7 +260,8 @@ def test_dense_levels_against_cosine_transform(size, bw, levels):
             want = idctn(f, type=2, norm="ortho")
             err = rel_l2(box_p, want)
             say("  level", l, n, "pressure rel l2", err)
-            assert err <= (1e-7 if prec != SOLVE_FP32 else 6e-8 * max(1.0, max(n) / np.pi) ** 2 + 1e-6)
+            noise = 20 + 40 * (max(n) / np.pi) ** 2 / np.sqrt(np.prod(n))
+            assert err <= (1e-7 if prec != SOLVE_FP32 else 6e-8 * noise)
     g.close()
 
 
