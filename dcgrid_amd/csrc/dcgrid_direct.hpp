@@ -20,7 +20,8 @@
 // the V-cycles of such a level (seven to nine, to 1e-8) it leaves one step at 1e-13: a projection of
 // 256 x 128 x 256 cells on three dense levels 6.24 -> 0.96 ms, of 512 x 128 x 512 on four 19.2 -> 4.1 ms,
 // of 512^3 cells in 32768 blocks of 8^3 (two of four levels dense) 4.82 -> 2.19 ms. In FP32 throughout, four to five
-// steps stall where the V-cycles' seven to nine did.
+// steps stall where the V-cycles' seven to nine did, at the rounding of the residual: over 192 levels of 17 grids
+// the pressure's error against 64 bits is 1.03 +- 0.04 times theirs (they fail on 40 more, which this solves).
 #pragma once
 
 #include "dcgrid_solve.hpp"
@@ -67,7 +68,9 @@ struct DctArgs {
   const SolveCtl* ctl;
 };
 static constexpr int kDctThreads = 512;
-// Longest axis: a tile of 16 lines is 144 KB at 1024 entries in FP64.
+// Longest axis: a tile of 16 lines is 144 KB at 1024 entries in FP64. Beyond 512 cells, with these tiles,
+// the direct solve is still 1.25x (1024 x 8 x 8 cells) to 9x (640 x 640 x 64) faster than the V-cycles in mixed
+// arithmetic (1024 x 256 x 1024 on two levels 118 -> 54 ms), and up to 512 3.3x to 10x.
 static constexpr int kDctMaxAxis = 1024;
 // LDS row of NC lines. The pad spreads a fragment's four rows over the banks.
 template <int NC>

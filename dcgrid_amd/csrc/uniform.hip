@@ -350,8 +350,8 @@ __global__ void __launch_bounds__(256) k_u_prolongate(float* __restrict__ pre, U
 // A single half-sweep of a grid that fits the caches is a launch (about 2.5 us) and a round trip to the
 // other XCDs' results for 0.2 us of work, and of a large one 12 B of HBM per cell: several sweeps of a
 // tile in registers share both. Measured (MI355X, k_u_jacobi -> k_u_sweeps, whole projections): 64^3 with
-// 100 sweeps 283 -> 161 us, 128^3 with 40 sweeps 336 -> 233 us, 320 x 256 x 384 with 10 sweeps 1507 ->
-// 940 us, multilevel 857 -> 657 us.
+// 100 sweeps 294 -> 157 us, 128^3 with 40 sweeps 312 -> 210 us, 320 x 256 x 384 with 10 sweeps 1490 ->
+// 840 us, multilevel 818 -> 579 us. Thin domains keep k_u_jacobi (sweepsFused).
 // A workgroup takes 64 x TY x TZ cells grown by K cells in y and z and, on a level wider than a
 // wavefront, in x. A wavefront is a row of 64 cells along x and keeps the rows of one y in
 // registers: x neighbours come by DPP, z neighbours from the same thread, y neighbours from LDS.
@@ -735,7 +735,7 @@ struct UniformSim : SimBase {
   // the prolonged pressure of the coarser level. Chunks of at most 4 sweeps a launch pass their
   // results through scratch (the advected velocity's second buffer, free between the advections);
   // the last one writes the last sweep to the pressure and the one before to t_pressure.
-  // Tiles: 4 x 4 in (y, z) while these are at most two per CU, so that every CU has one (64^3, 100
+  // Tiles (pairs of figures from one run each): 4 x 4 in (y, z) while these are at most two per CU, so that every CU has one (64^3, 100
   // sweeps: 4 x 4 161 us, 8 x 8 232 us); larger ones beyond, where the halo's redundant rows cost more
   // (128^3, 40 sweeps: 391 against 233 us; 96 x 100 x 104: 215 against 158 us). Five sweeps a launch
   // measured slower than four (128^3: 316 us), three about equal. Two sweeps (a level of the
